@@ -1,0 +1,89 @@
+"""The any-shape GEMM kernels at the edges of their tiles, against the CPU oracle.
+
+Every compiled variant (plan family 6) in both layouts and types, at sizes one below, at and above
+its tile, row segment (128 bytes of k) and chunk (16 bytes) boundaries, through operands aligned
+to one element only. Bounds: f32 sums of K products in [-1, 1] in any order stay within
+K * 2^-24 * sum|a b| of the exact sum, Frobenius about sqrt(K) * 2^-24 (2e-6 at K = 1100), gate 1e-5; f16
+results add one rounding to half (2^-11 relative at most, 2.1e-4 Frobenius), gate 1e-3.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import _oracle as O
+from test_gpu_gemm import f16_inputs, frob
+
+pytestmark = pytest.mark.gpu
+
+VARIANTS = [0, 2, 3, 4, 5, 6, 7, 8, 9, 10]
+F16_ONLY = (5, 6)
+# ragged around 64/128/256 tiles; K below a chunk, across a chunk, across segments and k groups
+SHAPES = [(1, 1, 1), (1, 3, 2), (5, 7, 3), (16, 64, 64), (17, 65, 63), (63, 33, 9), (65, 129, 257), (130, 255, 72),
+          (257, 260, 1091)]
+
+
+def run(uk, A, B, dtype, layout, variant, off):
+    """One launch with every operand `off` elements past a 256-byte boundary."""
+    M, K = A.shape
+    N = B.shape[0] if layout == "TN" else B.shape[1]
+    es = A.itemsize
+    d = uk.make_desc("gemm", [M, N, K], dtype=dtype, layout=layout)
+    p = uk.Plan()
+    p.family, p.variant = 6, variant
+    guard = 64
+    bufs = []
+    for a in (A, B):
+        flat = np.zeros(a.size + off, a.dtype)
+        flat[off:] = a.ravel()
+        bufs.append(uk.DeviceBuffer.from_array(flat))
+    out = uk.DeviceBuffer((M * N + off + guard) * es)
+    out.fill(0xFF)
+
+    class At:
+        def __init__(self, b):
+            self.ptr = C.c_void_p(b.ptr.value + off * es)
+
+    uk.launch(d, [At(b) for b in bufs], At(out), plan=p)
+    flat = out.download(A.dtype, (M * N + off + guard,)).view(np.uint16 if es == 2 else np.uint32)
+    edge = np.iinfo(flat.dtype).max
+    assert (flat[:off] == edge).all() and (flat[off + M * N:] == edge).all()  # nothing stored outside C
+    return flat[off:off + M * N].reshape(M, N).view(A.dtype)
+
+
+@pytest.mark.parametrize("layout", ["TN", "NT"])
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("dtype", ["fp16", "fp32"])
+def test_edges(gpu, dtype, variant, layout):
+    if dtype == "fp32" and variant in F16_ONLY:
+        pytest.skip("compiled for f16 only")
+    for i, (M, N, K) in enumerate(SHAPES):
+        if dtype == "fp16":
+            A, B = f16_inputs(M, N, K, 900 + i, tn=(layout == "TN"))
+            R = O.gemm_f16q(A, B, layout == "TN")
+        else:
+            A = O.uniform(M * K, 910 + i, -1.0, 1.0).reshape(M, K)
+            B = O.uniform(N * K, 920 + i, -1.0, 1.0).reshape((N, K) if layout == "TN" else (K, N))
+            R = O.gemm_f32(A, B, layout == "TN")
+        got = run(gpu, A, B, dtype, layout, variant, off=i % 4)
+        if dtype == "fp16":
+            got = O.f16_to_f32(got)
+        assert frob(got, R) <= (1e-3 if dtype == "fp16" else 1e-5), (M, N, K)
+
+
+@pytest.mark.parametrize("layout", ["TN", "NT"])
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_non_finite_values_stay_in_their_rows_and_columns(gpu, variant, layout):
+    # K = 70 leaves a partial segment and N, M partial tiles: what lies past an edge must not reach a
+    # sum (0 * inf is NaN). One infinity in the last row of A and one NaN in the last column of B.
+    M, N, K = 35, 37, 70
+    A, B = f16_inputs(M, N, K, 77)
+    A, B = O.f16_to_f32(A), O.f16_to_f32(B)
+    A[M - 1, K - 1] = np.inf
+    B[N - 1, 0] = np.nan
+    Ah, Bh = O.f16_bits(A), O.f16_bits(B if layout == "TN" else np.ascontiguousarray(B.T))
+    got = O.f16_to_f32(run(gpu, Ah, Bh, "fp16", layout, variant, off=1))
+    want = A.astype(np.float64) @ B.T.astype(np.float64)
+    assert np.isnan(got[:, N - 1]).all()
+    assert np.array_equal(got[M - 1, :N - 1], want[M - 1, :N - 1].astype(np.float32))  # +-inf
+    assert frob(got[:M - 1, :N - 1], want[:M - 1, :N - 1]) <= 1e-3

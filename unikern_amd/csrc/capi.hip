@@ -369,8 +369,7 @@ int prepare(const uk_op_desc* d, const uk_plan* plan, const Hcs* h, KmlTree* t, 
     return UK_OK;
   }
   std::string err;
-  SolveLog log;
-  auto sol = solve(h ? *h : hcs_mi355x(), *t, &log, &err);
+  auto sol = solve(h ? *h : hcs_mi355x(), *t, nullptr, &err);
   if (!sol) return fail(UK_INFEASIBLE, "UNIKERN_ERROR what=infeasible reason=" + err);
   *p = *sol;
   return UK_OK;
@@ -1225,8 +1224,13 @@ int uk_solve(const char* hcs_json, const uk_op_desc* d, uk_plan* out, char* log,
   os << "SOLVE family=" << to_string(p->family) << " key=" << p->key << " predicted_us=" << p->predicted_us
      << " feasible=" << p->feasible << " why=" << p->why;
   for (const auto& r : sl.rejected) os << "\n  rejected " << r;
-  for (const auto& [us, key] : sl.ranked) os << "\n  candidate " << key << " predicted_us=" << us;
-  put(os.str(), log, cap);
+  std::string text = os.str();
+  for (const auto& [us, key] : sl.ranked) {
+    char num[32];
+    std::snprintf(num, sizeof num, "%g", us);
+    text.append("\n  candidate ").append(key).append(" predicted_us=").append(num);
+  }
+  put(text, log, cap);
   return UK_OK;
 }
 

@@ -110,9 +110,12 @@ std::optional<Plan> pick(std::vector<Cand>& cs, const char* family_name, SolveLo
   for (const Cand& c : cs)
     if (c.cost < best->cost || (c.cost == best->cost && c.plan.key < best->plan.key)) best = &c;
   if (log) {
-    for (const Cand& c : cs)
-      log->ranked.emplace_back(c.cost, std::string(c.plan.key) + " family=" + std::to_string(int(c.plan.family)) +
-                                           " variant=" + std::to_string(c.plan.variant));
+    log->ranked.reserve(cs.size());
+    for (const Cand& c : cs) {
+      char tail[48];
+      std::snprintf(tail, sizeof tail, " family=%d variant=%d", int(c.plan.family), c.plan.variant);
+      log->ranked.emplace_back(c.cost, c.plan.key + tail);
+    }
     std::sort(log->ranked.begin(), log->ranked.end());
   }
   Plan p = best->plan;
@@ -197,6 +200,9 @@ std::optional<Plan> solve_rows(const Hcs& h, const KmlTree& t, const Shape& s, S
 
 // ---------------------------------------------------------------------------------------
 constexpr double kGemmF32Eff = 0.72;  // gemm_f32_kernel's fraction of the f32 MFMA rate (calibrated at 1024^3)
+
+// The shortest time measured for any launch of kernels/gemm_any.hip.
+constexpr double kGemmAnyFloorUs = 4.4;
 
 std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
   const double peak_tflops = t.dtype == DType::F16 ? (h.peak_f16_mfma_tflops > 0 ? h.peak_f16_mfma_tflops : h.flops_gflops * 1e-3)
@@ -304,23 +310,74 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
       cs.push_back(c);
     }
   }
-  {
+  const double stream_floor_us = launch_us(h) + double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3 * kStreamEff);
+  // The work constants were fitted on a part of 256 CUs at these dense matrix-core peaks.
+  const bool f16 = t.dtype == DType::F16, tn = t.layout == Layout::TN;
+  const double fit_scale =
+      (f16 ? 2516.5824 : 157.2864) / 256.0 / (peak_tflops * mfma_clock_scale(h) / double(cus(h)));
+  cs.reserve(cs.size() + kNumGemmAnyVariants);
+  for (const GemmAnyVariant& entry : kGemmAnyVariants) {
+    const GemmAnyVariant& v = entry.id == 0 && s.M <= 64 && s.N <= 64 ? gemm_any_variant(7) : entry;
+    if (v.f16_only && !f16) continue;
+    const int64_t slab = f16 ? 64 : 32;  // k of one 128-byte row segment
+    char key[64];
+    int64_t wgs, iters, lds;
+    int resident = v.resident;
     Cand c;
+    if (v.mt == 0) {
+      std::snprintf(key, sizeof key, "gemm_tile:%dx%d,k%d", v.bm, v.bn, v.ks);
+      wgs = ((s.M + v.bm - 1) / v.bm) * ((s.N + v.bn - 1) / v.bn);
+      iters = (s.K + v.ks * slab - 1) / (v.ks * slab);
+      lds = int64_t(2) * v.ks * (v.bm + v.bn) * 128;
+      c.plan.tile_m = v.bm;
+      c.plan.tile_n = v.bn;
+      c.plan.tile_k = int(v.ks * slab);
+      c.plan.threads = v.wm * v.wn * v.ks * 64;
+    } else {
+      const int waves = tn ? v.waves : gemm_skinny_nt_waves(v.waves);
+      const int cols = tn ? 16 * v.nt : 64;
+      std::snprintf(key, sizeof key, "gemm_skinny:%dx%d,w%d", 16 * v.mt, cols, waves);
+      wgs = ((s.M + 16 * v.mt - 1) / (16 * v.mt)) * ((s.N + cols - 1) / cols);
+      const int64_t step = tn ? slab : slab / 2;
+      iters = ((s.K + step - 1) / step + waves - 1) / waves;
+      lds = int64_t(waves) * v.mt * (cols / 16) * 1024;
+      resident = std::max(1, 16 / waves);
+      c.plan.tile_m = 16 * v.mt;
+      c.plan.tile_n = cols;
+      c.plan.tile_k = int(step);
+      c.plan.threads = waves * 64;
+      c.plan.split_k = waves;
+    }
+    // The kernel any shape falls back to is offered whatever the description says of LDS.
+    if (entry.id != 0 && lds > lds_block(h)) {
+      reject(log, std::string(key) + " violates LDS " + std::to_string(lds) + " <= " + std::to_string(lds_block(h)));
+      continue;
+    }
+    const double work = (f16 ? v.work_f16 : v.work_f32) * (tn ? 1.0 : v.nt_factor) * fit_scale;
+    const int64_t slots = int64_t(cus(h)) * resident;
+    const int64_t full = wgs / slots, rest = wgs % slots;
+    const double last = rest ? std::max(v.lat_us, double((rest + cus(h) - 1) / cus(h)) * work) : 0.0;
+    const double rounds_us =
+        v.fixed_us + (double(iters) + v.tail) * (double(full) * std::max(v.lat_us, resident * work) + last);
+    // No launch is shorter than its dispatch and one chain of memory latencies (kGemmAnyFloorUs), and
+    // none beats the streaming rate of its operands.
+    c.cost = std::max({kGemmAnyFloorUs, rounds_us, stream_floor_us});
     c.plan.family = Family::GemmGeneric;
-    c.plan.variant = 0;
-    c.plan.tile_m = c.plan.tile_n = kGemmGenericTile;
-    c.plan.tile_k = 16;
-    c.plan.threads = 256;
-    c.plan.grid = ((s.M + 63) / 64) * ((s.N + 63) / 64);
-    c.plan.key = "gemm_generic:64x64x16";
-    c.plan.why = "bounds-checked 64x64 MFMA tiles (any shape and layout)";
-    // Measured at the BASELINE shapes (element-wise staging, one 64x64 tile per workgroup):
-    // 1.5% of the f16 MFMA peak at 4096^3, 9% of the f32 peak at 1024^3.
-    const double eff = t.dtype == DType::F16 ? 0.016 : 0.09;
-    c.cost = launch_us(h) + flops / (peak_tflops * 1e6 * eff * mfma_clock_scale(h)) + 1.0;
-    cs.push_back(c);
+    c.plan.variant = entry.id;
+    c.plan.grid = wgs;
+    c.plan.key = key;
+    if (entry.id == 0) {
+      c.plan.key = "gemm_generic:64x64x16";  // x16: k of one step of f32 fragments
+      c.plan.tile_m = c.plan.tile_n = 64;
+      c.plan.tile_k = 16;
+    }
+    cs.push_back(std::move(c));
   }
-  return pick(cs, "gemm", log, err);
+  auto best = pick(cs, "gemm", log, err);
+  if (best && best->family == Family::GemmGeneric && best->variant != 1)
+    best->why = std::to_string(best->grid) + " workgroups of " + std::to_string(best->threads) +
+                " threads, any shape, layout and element alignment";
+  return best;
 }
 
 // ---------------------------------------------------------------------------------------

@@ -1,7 +1,7 @@
 // GEMM on gfx950 matrix cores.
 //
 // Replaces the reference's SIMT uk_gemm / uk_gemm_h (src/codegen_hip.cpp:1089-1120,
-// :1777-1808), which convert to f32 in LDS and run scalar FMAs. Eight kernels:
+// :1777-1808), which convert to f32 in LDS and run scalar FMAs. The kernels:
 //
 // gemm_f16_tn_kernel — the hot path: C[M][N] f16 = A[M][K] f16 . B^T, B stored [N][K]
 //   (column-major B: both operands K-contiguous), f32 accumulate in v_mfma_f32_32x32x16_f16.
@@ -59,9 +59,8 @@
 //   k = 8q + 4 + e on lanes 32-63 (any assignment of k to MFMA steps gives the same sum when A
 //   and B agree). The two halves' accumulators add in LDS in a fixed order.
 //
-// gemm_generic_kernel — any M, N, K, either B layout, f16 or f32 inputs: 64x64 tiles,
-//   bounds-checked element loads, MFMA 32x32x16 f16 or 32x32x2 f32. Used for shapes the
-//   fast kernels' divisibility predicates reject.
+// Shapes that the divisibility predicates of these kernels reject, and the other layouts and types,
+// run on the kernels of gemm_any.hip.
 #include <type_traits>
 #include <utility>
 
@@ -1431,60 +1430,6 @@ __global__ void __launch_bounds__(512)
   }
 }
 
-// ---------------------------------------------------------------------------------------
-// Generic MFMA GEMM: 64x64 tile, 4 wavefronts (2x2 of 32x32), BK = 16, bounds-checked.
-// T = _Float16 or float inputs; TO = output type; BT: B stored [N][K] (TN) else [K][N] (NT).
-// ---------------------------------------------------------------------------------------
-template <typename T, typename TO, bool BT>
-__global__ void __launch_bounds__(256)
-    gemm_generic_kernel(const T* __restrict__ A, const T* __restrict__ B, TO* __restrict__ C, int M, int N, int K) {
-  constexpr int BKg = 16;
-  __shared__ __attribute__((aligned(16))) T As[64][BKg];
-  __shared__ __attribute__((aligned(16))) T Bs[64][BKg];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = wave >> 1, wn = wave & 1;
-  f32x16 acc = f32x16{};
-  for (int k0 = 0; k0 < K; k0 += BKg) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int idx = tid * 4 + e;
-      const int r = idx / BKg, kk = idx % BKg;
-      const int gm = m0 + r, gk = k0 + kk;
-      As[r][kk] = (gm < M && gk < K) ? A[(int64_t)gm * K + gk] : T(0);
-      if (BT) {
-        const int gn = n0 + r;
-        Bs[r][kk] = (gn < N && gk < K) ? B[(int64_t)gn * K + gk] : T(0);
-      } else {
-        const int kr = idx / 64, nn = idx % 64;
-        const int gk2 = k0 + kr, gn = n0 + nn;
-        Bs[nn][kr] = (gn < N && gk2 < K) ? B[(int64_t)gk2 * N + gn] : T(0);
-      }
-    }
-    __syncthreads();
-    if constexpr (sizeof(T) == 2) {
-      const f16x8 a = *reinterpret_cast<const f16x8*>(&As[wm * 32 + (lane & 31)][(lane >> 5) * 8]);
-      const f16x8 b = *reinterpret_cast<const f16x8*>(&Bs[wn * 32 + (lane & 31)][(lane >> 5) * 8]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc, 0, 0, 0);
-    } else {
-#pragma unroll
-      for (int s = 0; s < BKg / 2; ++s) {
-        const float a = As[wm * 32 + (lane & 31)][2 * s + (lane >> 5)];
-        const float b = Bs[wn * 32 + (lane & 31)][2 * s + (lane >> 5)];
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  // D[i][j]: lane -> column j = lane & 31, rows i = 8*(r/4) + 4*(lane>>5) + r%4.
-  const int n = n0 + wn * 32 + (lane & 31);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + wm * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-    if (m < M && n < N) C[(int64_t)m * N + n] = (TO)acc[r];
-  }
-}
-
 }  // namespace uk::kern
 
 namespace uk {
@@ -1592,50 +1537,22 @@ bool gemm_f32_tiled_supported(int64_t M, int64_t N, int64_t K) {
 
 hipError_t launch_gemm_generic(int variant, DType dt, Layout lay, const void* A, const void* B, void* C, int64_t M,
                                int64_t N, int64_t K, hipStream_t s) {
-  if (M <= 0 || N <= 0 || K <= 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return hipErrorInvalidValue;
+  if (variant != 1) return launch_gemm_any(variant, dt, lay, A, B, C, M, N, K, s);
+  // gemm_f32_kernel: f32, 64-multiples, 16-byte aligned operands
   if (lay != Layout::NT && lay != Layout::TN) return hipErrorInvalidValue;
-  if ((M + 63) / 64 > 65535) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  const bool bt = lay == Layout::TN;
-  if (variant == 1) {  // gemm_f32_kernel: f32, 64-multiples, 16-byte aligned operands
-    if (dt != DType::F32 || !gemm_f32_tiled_supported(M, N, K)) return hipErrorInvalidValue;
-    if ((((uintptr_t)A) | ((uintptr_t)B) | ((uintptr_t)C)) & 15) return hipErrorInvalidValue;
-    auto a = static_cast<const float*>(A);
-    auto b = static_cast<const float*>(B);
-    auto c = static_cast<float*>(C);
-    const int tm = int(M / 64), tn = int(N / 64);
-    if (int64_t(tm) * tn > INT32_MAX) return hipErrorInvalidValue;
-    const dim3 g1((unsigned)(tm * tn));
-    if (bt)
-      hipLaunchKernelGGL((kern::gemm_f32_kernel<true>), g1, dim3(512), 0, s, a, b, c, (int)M, (int)N, (int)K, tm, tn);
-    else
-      hipLaunchKernelGGL((kern::gemm_f32_kernel<false>), g1, dim3(512), 0, s, a, b, c, (int)M, (int)N, (int)K, tm, tn);
-    return hipGetLastError();
-  }
-  if (variant != 0) return hipErrorInvalidValue;
-  if (dt == DType::F16) {
-    auto a = static_cast<const _Float16*>(A);
-    auto b = static_cast<const _Float16*>(B);
-    auto c = static_cast<_Float16*>(C);
-    if (bt)
-      hipLaunchKernelGGL((kern::gemm_generic_kernel<_Float16, _Float16, true>), grid, dim3(256), 0, s, a, b, c,
-                         (int)M, (int)N, (int)K);
-    else
-      hipLaunchKernelGGL((kern::gemm_generic_kernel<_Float16, _Float16, false>), grid, dim3(256), 0, s, a, b, c,
-                         (int)M, (int)N, (int)K);
-  } else if (dt == DType::F32) {
-    auto a = static_cast<const float*>(A);
-    auto b = static_cast<const float*>(B);
-    auto c = static_cast<float*>(C);
-    if (bt)
-      hipLaunchKernelGGL((kern::gemm_generic_kernel<float, float, true>), grid, dim3(256), 0, s, a, b, c, (int)M,
-                         (int)N, (int)K);
-    else
-      hipLaunchKernelGGL((kern::gemm_generic_kernel<float, float, false>), grid, dim3(256), 0, s, a, b, c, (int)M,
-                         (int)N, (int)K);
-  } else {
-    return hipErrorInvalidValue;
-  }
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || (M + 63) / 64 > 65535) return hipErrorInvalidValue;
+  if (dt != DType::F32 || !gemm_f32_tiled_supported(M, N, K)) return hipErrorInvalidValue;
+  if ((((uintptr_t)A) | ((uintptr_t)B) | ((uintptr_t)C)) & 15) return hipErrorInvalidValue;
+  auto a = static_cast<const float*>(A);
+  auto b = static_cast<const float*>(B);
+  auto c = static_cast<float*>(C);
+  const int tm = int(M / 64), tn = int(N / 64);
+  if (int64_t(tm) * tn > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 g1((unsigned)(tm * tn));
+  if (lay == Layout::TN)
+    hipLaunchKernelGGL((kern::gemm_f32_kernel<true>), g1, dim3(512), 0, s, a, b, c, (int)M, (int)N, (int)K, tm, tn);
+  else
+    hipLaunchKernelGGL((kern::gemm_f32_kernel<false>), g1, dim3(512), 0, s, a, b, c, (int)M, (int)N, (int)K, tm, tn);
   return hipGetLastError();
 }
 

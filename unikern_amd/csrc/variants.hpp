@@ -103,8 +103,43 @@ constexpr GemmF16Variant kGemmF16Variants[] = {
 };
 constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Variants[0]);
 
-// Generic MFMA GEMM (any M, N, K; NT or TN; fp16 or fp32 inputs): 64x64 tiles, 4 waves.
-constexpr int kGemmGenericTile = 64;
+// GEMM of any M, N, K, either B layout, fp16 or fp32, element-aligned operands (kernels/gemm_any.hip).
+// tile (mt == 0): a bm x bn tile per workgroup, wm x wn wavefronts per k group and ks k groups, each
+// multiplying its own 128-byte k segment of the rows. skinny (mt > 0): 16 mt rows of A per workgroup,
+// `waves` wavefronts splitting k over 16 nt columns of B ([N][K]) or 64 ([K][N], with twice the
+// wavefronts up to 16), operands straight into registers.
+// The cost of a variant is fixed_us + (iterations + tail) * sum over rounds of max(lat_us, n * work),
+// with n the workgroups a CU holds in that round: lat_us is one iteration's load latency, work its
+// share of the CU's time (work_f16 / work_f32, times nt_factor where B is [K][N]), tail the fold and
+// stores in iterations. Fitted over 419 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every
+// variant measured at each, both types and layouts): the pick's time is 3% over the fastest variant's
+// on average, 71% at worst (a 67-column product).
+// The 64x64 variant 0 is the one any plan falls back to; a single tile of it (M, N <= 64) runs as
+// variant 7, whose 16-column workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
+// id: the plan's variant number (1 is gemm_f32_kernel). resident: workgroups per CU by LDS and registers.
+struct GemmAnyVariant {
+  int id, bm, bn, wm, wn, ks, mt, nt, waves, unroll, resident, f16_only;
+  double lat_us, work_f16, work_f32, nt_factor, fixed_us, tail;
+};
+constexpr GemmAnyVariant kGemmAnyVariants[] = {
+    {0, 64, 64, 2, 2, 1, 0, 0, 0, 0, 4, 0, 0.485, 0.314, 0.661, 1.144, 3.461, 0.176},
+    {2, 64, 64, 2, 2, 2, 0, 0, 0, 0, 2, 0, 0.540, 0.618, 1.172, 1.186, 2.863, 0.700},
+    {3, 64, 64, 2, 2, 4, 0, 0, 0, 0, 1, 0, 0.600, 1.162, 2.450, 1.163, 1.079, 1.597},
+    {4, 128, 64, 2, 2, 1, 0, 0, 0, 0, 3, 0, 0.551, 0.576, 1.164, 1.253, 3.832, 0.000},
+    {5, 256, 128, 4, 2, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.157, 0.000, 1.131, 3.451, 0.203},
+    {6, 256, 256, 2, 4, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.751, 0.000, 1.404, 4.475, 0.000},
+    {7, 16, 16, 0, 0, 0, 1, 1, 8, 4, 2, 0, 0.869, 0.805, 0.808, 2.364, 1.083, 0.088},
+    {8, 16, 32, 0, 0, 0, 1, 2, 4, 4, 4, 0, 0.566, 0.630, 0.667, 1.503, 1.285, 0.379},
+    {9, 32, 32, 0, 0, 0, 2, 2, 8, 2, 2, 0, 0.600, 1.494, 1.838, 1.563, 1.140, 0.400},
+    {10, 32, 64, 0, 0, 0, 2, 4, 8, 2, 2, 0, 0.600, 2.501, 3.304, 0.893, 0.000, 0.599},
+};
+constexpr int kNumGemmAnyVariants = sizeof(kGemmAnyVariants) / sizeof(kGemmAnyVariants[0]);
+constexpr const GemmAnyVariant& gemm_any_variant(int id) {
+  for (const GemmAnyVariant& v : kGemmAnyVariants)
+    if (v.id == id) return v;
+  return kGemmAnyVariants[0];
+}
+constexpr int gemm_skinny_nt_waves(int waves) { return 2 * waves <= 16 ? 2 * waves : 16; }
 
 // Q8_0 skinny GEMM: a workgroup owns 16 nt weight rows; each of its wavefronts copies `pairs`
 // block pairs of those rows per round into its own LDS area (nt * pairs * 1088 bytes) and

@@ -30,7 +30,7 @@ KERNELS = {
     "copy": re.compile(r"rows_kernel<64, 16, 3[,>]"),
     "gemm_f16": re.compile(r"gemm_f16_(tn|pp|w4|w4s|w4k|w4k16)_kernel"),
     "gemm_f32": re.compile(r"gemm_f32_kernel"),
-    "gemm_generic": re.compile(r"gemm_generic_kernel"),
+    "gemm_generic": re.compile(r"gemm_any_kernel|gemm_skinny_(tn|nt)_kernel"),
     "conv": re.compile(r"conv_igemm_kernel|conv_tile_kernel|conv_lds_kernel|conv_lds16_kernel"),
     "q8_0": re.compile(r"q8_0_gemm_kernel|q8_0_gemv_kernel"),
 }
