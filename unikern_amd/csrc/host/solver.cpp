@@ -310,11 +310,13 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
       cs.push_back(c);
     }
   }
-  const double stream_floor_us = launch_us(h) + double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3 * kStreamEff);
   // The work constants were fitted on a part of 256 CUs at these dense matrix-core peaks.
   const bool f16 = t.dtype == DType::F16, tn = t.layout == Layout::TN;
   const double fit_scale =
       (f16 ? 2516.5824 : 157.2864) / 256.0 / (peak_tflops * mfma_clock_scale(h) / double(cus(h)));
+  const double roof_us =
+      launch_us(h) + std::max(double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
+                              flops / (peak_tflops * 1e6 * mfma_clock_scale(h) * (f16 ? kGemmAnyPeakF16 : kGemmAnyPeakF32)));
   cs.reserve(cs.size() + kNumGemmAnyVariants);
   for (const GemmAnyVariant& entry : kGemmAnyVariants) {
     const GemmAnyVariant& v = entry.id == 0 && s.M <= 64 && s.N <= 64 ? gemm_any_variant(7) : entry;
@@ -353,15 +355,16 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
       reject(log, std::string(key) + " violates LDS " + std::to_string(lds) + " <= " + std::to_string(lds_block(h)));
       continue;
     }
-    const double work = (f16 ? v.work_f16 : v.work_f32) * (tn ? 1.0 : v.nt_factor) * fit_scale;
+    const double work = (f16 ? v.work_f16 : v.work_f32) * (tn ? 1.0 : v.nt_factor) *
+                        ((tn ? s.K : s.N) % (slab / 8) ? v.unaligned : 1.0) * fit_scale;
     const int64_t slots = int64_t(cus(h)) * resident;
     const int64_t full = wgs / slots, rest = wgs % slots;
     const double last = rest ? std::max(v.lat_us, double((rest + cus(h) - 1) / cus(h)) * work) : 0.0;
     const double rounds_us =
         v.fixed_us + (double(iters) + v.tail) * (double(full) * std::max(v.lat_us, resident * work) + last);
     // No launch is shorter than its dispatch and one chain of memory latencies (kGemmAnyFloorUs), and
-    // none beats the streaming rate of its operands.
-    c.cost = std::max({kGemmAnyFloorUs, rounds_us, stream_floor_us});
+    // none beats the streaming rate of its operands or the matrix cores' sustained rate.
+    c.cost = std::max({kGemmAnyFloorUs, rounds_us, roof_us});
     c.plan.family = Family::GemmGeneric;
     c.plan.variant = entry.id;
     c.plan.grid = wgs;

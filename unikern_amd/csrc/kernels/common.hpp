@@ -52,6 +52,19 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(readlane(v, 0), readlane(v, 32));
 }
 
+// 16 bytes at any element-aligned global address (one unaligned 128-bit load).
+__device__ __forceinline__ u32x4 any_load16(const void* p) {
+  u32x4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// Workgroup barrier that waits for this wavefront's LDS operations only: global loads into registers
+// stay in flight across it (the compiler waits for them where their values are used).
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
 }  // namespace uk::kern

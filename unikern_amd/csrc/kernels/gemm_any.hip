@@ -7,21 +7,26 @@
 // Two forms (kGemmAnyVariants lists the compiled ones and their costs):
 //
 // gemm_any_kernel: a BM x BN tile per workgroup, operands staged through registers into two LDS
-//   slots, the next k step's loads in flight while the current one is multiplied, one barrier per
-//   step. Registers (not direct-to-LDS copies) because rows of any length start at any address: the
-//   unaligned 128-bit loads need no special case, only chunks that cross the end of a row do, and B
-//   stored [K][N] is transposed on its way (v_perm on pairs of k). With S > 1, S groups of
+//   slots, one barrier per step of k. A step stores the next step's operands, loaded D steps ago,
+//   issues the loads that replace them and multiplies: the loads have D whole steps to land, and the
+//   barrier waits for LDS only. The loop has no branch around a load (past the end they repeat the last
+//   whole step; the partial step has loads of its own), because with one the compiler can no longer
+//   count the loads in flight and waits for all of them: storing after the multiply, with branches,
+//   256x256 took 117.5 us at 1000x11008x4096 (107 now) and 64x64 in two k groups 32.3 us at f32 NT
+//   1000^3 (24.8 now). Registers (not direct-to-LDS copies) because rows of any length start at any
+//   address: the unaligned 128-bit loads need no special case, only chunks that cross the end of a row
+//   do, and B stored [K][N] is transposed on its way (v_perm on pairs of k). With S > 1, S groups of
 //   wavefronts multiply S consecutive 128-byte segments and add their sums in LDS at the end: small
-//   grids then have S times the loads in flight. Bound by load latency below about two workgroups
-//   per CU and by the matrix pipe of two wavefronts per SIMD above.
+//   grids then have S times the loads in flight. Bound by load latency below about two workgroups per
+//   CU and by the matrix pipe of two wavefronts per SIMD above.
 // gemm_skinny_*_kernel: 16-32 rows of A. Wavefronts split k, each lane loads its fragments of both
 //   operands straight into registers (no LDS, no barrier until the partial sums are added), several
 //   steps' loads in flight. Bound by the stream of B.
 //
 // Measured against the bounds-checked 64x64x16 kernel these replaced (element loads, two barriers per
-// 16 k), one box, inputs rotating over three sets: f16 TN 1000x11008x4096 2683 -> 117.5 us (768
-// TFLOP/s; 256x256), 16x11008x4096 252 -> 24.1 us (3.8 TB/s; skinny), f16 NT 512x9728x2560 440 ->
-// 49.2 us (519 TFLOP/s; 256x128), f32 NT 1000^3 131 -> 32.4 us (62 TFLOP/s; 64x64 in two k groups),
+// 16 k), one box, inputs rotating over three sets: f16 TN 1000x11008x4096 2667 -> 106.7 us (846
+// TFLOP/s; 256x256), 16x11008x4096 251 -> 23.9 us (3.8 TB/s; skinny), f16 NT 512x9728x2560 440 ->
+// 47.0 us (543 TFLOP/s; 256x128), f32 NT 1000^3 131 -> 24.8 us (81 TFLOP/s; 64x64 in two k groups),
 // and against 64 bits the f32 sums are no further off (4.0e-7 against 5.7e-7).
 #include "../launch.hpp"
 #include "../variants.hpp"
@@ -31,13 +36,6 @@
 #include <utility>
 
 namespace uk::kern {
-
-// 16 bytes at any element-aligned global address (one unaligned 128-bit load).
-__device__ __forceinline__ u32x4 any_load16(const void* p) {
-  u32x4 v;
-  __builtin_memcpy(&v, p, 16);
-  return v;
-}
 
 // Elements [x, x + E) of a line of X elements at `line` (E = 16 / sizeof(T)), zero past the end.
 // A chunk that crosses the end reads the line's last E elements and shifts them down.
@@ -112,7 +110,7 @@ struct AnyCfg {
   static constexpr int kLds = kPipe > kRed ? (kPipe > kStage ? kPipe : kStage) : (kRed > kStage ? kRed : kStage);
 };
 
-template <typename T, int BM, int BN, int WM, int WN, int S, bool BT>
+template <typename T, int BM, int BN, int WM, int WN, int S, int D, bool BT>
 __global__ void __launch_bounds__(WM* WN* S * 64)
     gemm_any_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, int M, int N, int K, int tiles_m,
                     int tiles_n) {
@@ -168,53 +166,69 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   } else {
     brow[0] = B;
   }
+  // B stored [K][N] at the right edge (N >= E there): a chunk that crosses N is read as the row's last
+  // E columns and its own moved to their places when it is stored.
   const bool whole_n = BT || N - n0 >= BN;
+  const int nb = n0 + nc * E;
+  const int nl = N - nb >= E ? nb : N - E;
+  const int nshift = nb - nl < E ? (nb - nl) * (int)sizeof(T) * 8 : 0;
 
-  u32x4 ra[NA], rb[NB];
-  auto load = [&](int t) __attribute__((always_inline)) {
-    const int k0 = t * KT_ELEMS + kh * SLAB;
-    const bool whole = K - k0 >= SLAB && whole_n;
-    if (whole) {
+  // Whole steps of k, and a last partial one. Loads of whole step t into register set t % D; past the
+  // last they read it again: no branch, so the compiler waits for one step's loads by count while the
+  // next step's are in flight.
+  const int whole_steps = K / KT_ELEMS;
+  const bool tail = whole_steps * KT_ELEMS < K;
+  u32x4 ra[D][NA], rb[D][NB];
+  auto load = [&](auto set_c, int t) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value % D;
+    const int k0 = (t < whole_steps ? t : whole_steps - 1) * KT_ELEMS + kh * SLAB;
 #pragma unroll
-      for (int u = 0; u < NA; ++u) ra[u] = any_load16(arow[u] + k0 + cc * E);
-      if constexpr (BT) {
+    for (int u = 0; u < NA; ++u) ra[set][u] = any_load16(arow[u] + k0 + cc * E);
+    if constexpr (BT) {
 #pragma unroll
-        for (int u = 0; u < NB; ++u) rb[u] = any_load16(brow[u] + k0 + cc * E);
-      } else {
-#pragma unroll
-        for (int u = 0; u < NB; ++u) rb[u] = any_load16(B + (int64_t)(k0 + kg * NB + u) * N + n0 + nc * E);
-      }
+      for (int u = 0; u < NB; ++u) rb[set][u] = any_load16(brow[u] + k0 + cc * E);
     } else {
 #pragma unroll
-      for (int u = 0; u < NA; ++u) ra[u] = any_load16_edge(arow[u], k0 + cc * E, K);
+      for (int u = 0; u < NB; ++u) rb[set][u] = any_load16(B + (int64_t)(k0 + kg * NB + u) * N + nl);
+    }
+  };
+  auto load_tail = [&](u32x4(&ta)[NA], u32x4(&tb)[NB]) __attribute__((always_inline)) {
+    const int k0 = whole_steps * KT_ELEMS + kh * SLAB;
 #pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        if constexpr (BT) {
-          rb[u] = any_load16_edge(brow[u], k0 + cc * E, K);
-        } else {
-          const int k = k0 + kg * NB + u;
-          rb[u] = k < K ? any_load16_edge(B + (int64_t)k * N, n0 + nc * E, N) : u32x4{0, 0, 0, 0};
-        }
+    for (int u = 0; u < NA; ++u) ta[u] = any_load16_edge(arow[u], k0 + cc * E, K);
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if constexpr (BT) {
+        tb[u] = any_load16_edge(brow[u], k0 + cc * E, K);
+      } else {
+        const int k = k0 + kg * NB + u;
+        tb[u] = k < K ? any_load16(B + (int64_t)k * N + nl) : u32x4{0, 0, 0, 0};
       }
     }
   };
   // 16-byte chunk c of row r sits at c ^ ((r >> 1) & 7): fragment reads (16 rows at one chunk
   // column) spread over the banks.
-  auto store = [&](int slot) __attribute__((always_inline)) {
+  auto store = [&](u32x4(&sa)[NA], u32x4(&sb)[NB], auto slot_c) __attribute__((always_inline)) {
+    const int slot = slot_c;
     char* as = lds + (slot * S + kh) * Cfg::kSlot;
     char* bs = as + Cfg::kOpA;
 #pragma unroll
     for (int u = 0; u < NA; ++u) {
       const int r = u * (Cfg::kGroup / 8) + crow;
-      *reinterpret_cast<u32x4*>(as + r * 128 + ((cc ^ ((r >> 1) & 7)) << 4)) = ra[u];
+      *reinterpret_cast<u32x4*>(as + r * 128 + ((cc ^ ((r >> 1) & 7)) << 4)) = sa[u];
     }
     if constexpr (BT) {
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         const int r = u * (Cfg::kGroup / 8) + crow;
-        *reinterpret_cast<u32x4*>(bs + r * 128 + ((cc ^ ((r >> 1) & 7)) << 4)) = rb[u];
+        *reinterpret_cast<u32x4*>(bs + r * 128 + ((cc ^ ((r >> 1) & 7)) << 4)) = sb[u];
       }
     } else {
+      if (!whole_n) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+          sb[u] = __builtin_bit_cast(u32x4, (unsigned __int128)(__builtin_bit_cast(unsigned __int128, sb[u]) >> nshift));
+      }
 #pragma unroll
       for (int j = 0; j < E; ++j) {
         const int r = nc * E + j;
@@ -223,7 +237,7 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
           uint32_t o[NB / 2];
 #pragma unroll
           for (int p = 0; p < NB / 2; ++p)
-            o[p] = __builtin_amdgcn_perm(rb[2 * p + 1][j >> 1], rb[2 * p][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+            o[p] = __builtin_amdgcn_perm(sb[2 * p + 1][j >> 1], sb[2 * p][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
           const int kb = kg * NB * 2;  // byte of the row segment
           char* dst = bs + r * 128 + (((kb >> 4) ^ ((r >> 1) & 7)) << 4) + (kb & 15);
           if constexpr (NB == 4) *reinterpret_cast<u32x2*>(dst) = u32x2{o[0], o[1]};
@@ -231,8 +245,8 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
         } else {
           const int kb = kg * NB * 4;
           char* dst = bs + r * 128 + (((kb >> 4) ^ ((r >> 1) & 7)) << 4) + (kb & 15);
-          if constexpr (NB == 4) *reinterpret_cast<u32x4*>(dst) = u32x4{rb[0][j], rb[1][j], rb[2][j], rb[3][j]};
-          else *reinterpret_cast<u32x2*>(dst) = u32x2{rb[0][j], rb[1][j]};
+          if constexpr (NB == 4) *reinterpret_cast<u32x4*>(dst) = u32x4{sb[0][j], sb[1][j], sb[2][j], sb[3][j]};
+          else *reinterpret_cast<u32x2*>(dst) = u32x2{sb[0][j], sb[1][j]};
         }
       }
     }
@@ -245,7 +259,8 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int slot) __attribute__((always_inline)) {
+  auto multiply = [&](auto slot_c) __attribute__((always_inline)) {
+    const int slot = slot_c;
     const char* as = lds + (slot * S + kh) * Cfg::kSlot + (wm * (BM / WM) + fi) * 128;
     const char* bs = lds + (slot * S + kh) * Cfg::kSlot + Cfg::kOpA + (wn * (BN / WN) + fi) * 128;
 #pragma unroll
@@ -263,15 +278,51 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
     }
   };
 
-  const int KT = K / KT_ELEMS + (K % KT_ELEMS != 0);
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int t = 0; t < KT; ++t) {
-    if (t + 1 < KT) load(t + 1);
-    multiply(t & 1);
-    if (t + 1 < KT) store((t + 1) & 1);
-    __syncthreads();
+  // Step t: its operands sit in slot t % 2; the next step's, loaded D steps ago, go into the other slot
+  // (every wavefront passed the barrier after reading it), the loads of step t + 1 + D take their
+  // registers, and only then does it multiply. With D = 2 (tiles whose registers allow it) sets and
+  // slots are compile-time constants and the tail's loads, issued first, have registers of their own.
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  auto step = [&](auto set_c, auto slot_c, auto next_c, int t) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value % D;
+    store(ra[set], rb[set], next_c);
+    load(set_c, t + 1 + D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(slot_c);
+    lds_barrier();
+  };
+  u32x4 ta[D == 2 ? NA : 1], tb[D == 2 ? NB : 1];
+  if constexpr (D == 2) {
+    if (tail) load_tail(ta, tb);
+  }
+  if (whole_steps > 0) {
+    load(I0{}, 0);
+    if constexpr (D == 2) load(I1{}, 1);
+    store(ra[0], rb[0], I0{});
+    load(I0{}, D);
+    lds_barrier();
+    if constexpr (D == 2) {
+      int t = 0;
+      for (; t + 1 < whole_steps; t += 2) {
+        step(I1{}, I0{}, I1{}, t);
+        step(I0{}, I1{}, I0{}, t + 1);
+      }
+      if (t < whole_steps) step(I1{}, I0{}, I1{}, t);
+    } else {
+      for (int t = 0; t < whole_steps; ++t) step(I0{}, t & 1, (t + 1) & 1, t);
+    }
+  }
+  if (tail) {
+    if constexpr (D == 2) {
+      store(ta, tb, I0{});
+    } else {
+      load_tail(ra[0], rb[0]);
+      store(ra[0], rb[0], I0{});
+    }
+    lds_barrier();
+    multiply(I0{});
+    lds_barrier();
   }
 
   // k groups 1 .. S - 1 hand their sums to group 0, which adds them in order.
@@ -526,6 +577,9 @@ dim3 any_grid(int64_t wgs) {
   return wgs <= kRow ? dim3((unsigned)wgs) : dim3((unsigned)kRow, (unsigned)((wgs + kRow - 1) / kRow));
 }
 
+constexpr int kGemmAnyNarrow = 7;  // the skinny 16x32 entry
+static_assert(kGemmAnyVariants[kGemmAnyNarrow].id == 8 && kGemmAnyVariants[kGemmAnyNarrow].mt == 1, "a skinny variant");
+
 template <int I, typename T>
 hipError_t any_go(bool bt, const T* a, const T* b, T* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
   constexpr GemmAnyVariant v = kGemmAnyVariants[I];
@@ -533,10 +587,13 @@ hipError_t any_go(bool bt, const T* a, const T* b, T* c, int64_t M, int64_t N, i
     return hipErrorInvalidValue;
   } else if constexpr (v.mt == 0) {
     using Cfg = kern::AnyCfg<T, v.bm, v.bn, v.wm, v.wn, v.ks>;
+    // B stored [K][N] is read in 16-byte chunks of a row: narrower products run as skinny ones.
+    if (!bt && N * (int64_t)sizeof(T) < 16) return any_go<kGemmAnyNarrow, T>(bt, a, b, c, M, N, K, s);
     const int64_t tm = (M + v.bm - 1) / v.bm, tn = (N + v.bn - 1) / v.bn;
     if (tm * tn > INT32_MAX) return hipErrorInvalidValue;
-    auto* k = bt ? kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, true>
-                 : kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, false>;
+    constexpr int D = v.bm * v.bn >= 128 * 64 ? 1 : 2;  // registers for two load sets
+    auto* k = bt ? kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, true>
+                 : kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, false>;
     hipLaunchKernelGGL(k, any_grid(tm * tn), dim3(Cfg::kThreads), 0, s, a, b, c, (int)M, (int)N, (int)K, (int)tm,
                        (int)tn);
     return hipGetLastError();

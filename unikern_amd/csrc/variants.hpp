@@ -110,29 +110,31 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // wavefronts up to 16), operands straight into registers.
 // The cost of a variant is fixed_us + (iterations + tail) * sum over rounds of max(lat_us, n * work),
 // with n the workgroups a CU holds in that round: lat_us is one iteration's load latency, work its
-// share of the CU's time (work_f16 / work_f32, times nt_factor where B is [K][N]), tail the fold and
-// stores in iterations. Fitted over 419 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every
-// variant measured at each, both types and layouts): the pick's time is 3% over the fastest variant's
-// on average, 71% at worst (a 67-column product).
+// share of the CU's time (work_f16 / work_f32, times nt_factor where B is [K][N], times `unaligned`
+// where the rows of B are not whole 16-byte chunks), tail the fold and stores in iterations. Fitted
+// over 515 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every variant measured at each, both
+// types and layouts): the pick's time is about 2% over the fastest variant's on average. Whatever the
+// sum says, no variant has sustained more than kGemmAnyPeakF16 / F32 of the matrix-core peak.
 // The 64x64 variant 0 is the one any plan falls back to; a single tile of it (M, N <= 64) runs as
 // variant 7, whose 16-column workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
 // id: the plan's variant number (1 is gemm_f32_kernel). resident: workgroups per CU by LDS and registers.
 struct GemmAnyVariant {
   int id, bm, bn, wm, wn, ks, mt, nt, waves, unroll, resident, f16_only;
-  double lat_us, work_f16, work_f32, nt_factor, fixed_us, tail;
+  double lat_us, work_f16, work_f32, nt_factor, fixed_us, tail, unaligned;
 };
 constexpr GemmAnyVariant kGemmAnyVariants[] = {
-    {0, 64, 64, 2, 2, 1, 0, 0, 0, 0, 4, 0, 0.485, 0.314, 0.661, 1.144, 3.461, 0.176},
-    {2, 64, 64, 2, 2, 2, 0, 0, 0, 0, 2, 0, 0.540, 0.618, 1.172, 1.186, 2.863, 0.700},
-    {3, 64, 64, 2, 2, 4, 0, 0, 0, 0, 1, 0, 0.600, 1.162, 2.450, 1.163, 1.079, 1.597},
-    {4, 128, 64, 2, 2, 1, 0, 0, 0, 0, 3, 0, 0.551, 0.576, 1.164, 1.253, 3.832, 0.000},
-    {5, 256, 128, 4, 2, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.157, 0.000, 1.131, 3.451, 0.203},
-    {6, 256, 256, 2, 4, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.751, 0.000, 1.404, 4.475, 0.000},
-    {7, 16, 16, 0, 0, 0, 1, 1, 8, 4, 2, 0, 0.869, 0.805, 0.808, 2.364, 1.083, 0.088},
-    {8, 16, 32, 0, 0, 0, 1, 2, 4, 4, 4, 0, 0.566, 0.630, 0.667, 1.503, 1.285, 0.379},
-    {9, 32, 32, 0, 0, 0, 2, 2, 8, 2, 2, 0, 0.600, 1.494, 1.838, 1.563, 1.140, 0.400},
-    {10, 32, 64, 0, 0, 0, 2, 4, 8, 2, 2, 0, 0.600, 2.501, 3.304, 0.893, 0.000, 0.599},
+    {0, 64, 64, 2, 2, 1, 0, 0, 0, 0, 4, 0, 0.270, 0.297, 0.600, 1.255, 2.860, 1.045, 1.135},
+    {2, 64, 64, 2, 2, 2, 0, 0, 0, 0, 2, 0, 0.361, 0.531, 1.150, 1.120, 2.502, 1.396, 1.172},
+    {3, 64, 64, 2, 2, 4, 0, 0, 0, 0, 1, 0, 0.600, 1.346, 2.450, 1.050, 1.224, 1.315, 1.110},
+    {4, 128, 64, 2, 2, 1, 0, 0, 0, 0, 3, 0, 0.662, 0.473, 1.183, 1.020, 2.908, 0.854, 1.099},
+    {5, 256, 128, 4, 2, 1, 0, 0, 0, 0, 1, 1, 0.600, 0.926, 0.000, 1.096, 0.000, 4.178, 1.156},
+    {6, 256, 256, 2, 4, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.573, 0.000, 1.089, 0.000, 3.277, 1.138},
+    {7, 16, 16, 0, 0, 0, 1, 1, 8, 4, 2, 0, 0.720, 0.766, 0.794, 2.324, 1.485, 0.000, 1.147},
+    {8, 16, 32, 0, 0, 0, 1, 2, 4, 4, 4, 0, 0.608, 0.596, 0.649, 1.443, 1.606, 0.500, 1.237},
+    {9, 32, 32, 0, 0, 0, 2, 2, 8, 2, 2, 0, 0.600, 1.473, 1.933, 1.493, 0.951, 0.230, 1.171},
+    {10, 32, 64, 0, 0, 0, 2, 4, 8, 2, 2, 0, 0.600, 2.481, 3.245, 0.853, 0.494, 0.452, 1.189},
 };
+constexpr double kGemmAnyPeakF16 = 0.467, kGemmAnyPeakF32 = 0.80;
 constexpr int kNumGemmAnyVariants = sizeof(kGemmAnyVariants) / sizeof(kGemmAnyVariants[0]);
 constexpr const GemmAnyVariant& gemm_any_variant(int id) {
   for (const GemmAnyVariant& v : kGemmAnyVariants)
