@@ -160,7 +160,9 @@ __global__ void __launch_bounds__(WAVES * 64)
   auto issue_x = [&](int p0, f16x8 (&xa)[P], f16x8 (&xb)[P]) __attribute__((always_inline)) {
     if constexpr (XL > 0) {
       // Lanes 0-31 copy row 2t's slice, lanes 32-63 row 2t + 1's (16 bytes each, in order).
-      const int64_t po = 64 * (p0 < npairs ? p0 : 0) + (lane & 31) * 8;
+      // A slice is four pairs; lanes of pairs past K/64 read pair 0 (never multiplied), not past the row.
+      const int pr = p0 + ((lane & 31) >> 3);
+      const int64_t po = 64 * (pr < npairs ? pr : 0) + (lane & 7) * 8;
       for (int t = 0; 2 * t < xr; ++t) {
         const int r = 2 * t + (lane >> 5);
         if (r < xr)
