@@ -87,3 +87,36 @@ def test_non_finite_values_stay_in_their_rows_and_columns(gpu, variant, layout):
     assert np.isnan(got[:, N - 1]).all()
     assert np.array_equal(got[M - 1, :N - 1], want[M - 1, :N - 1].astype(np.float32))  # +-inf
     assert frob(got[:M - 1, :N - 1], want[:M - 1, :N - 1]) <= 1e-3
+
+
+Q8_TILES = [11, 12, 13]  # 32x64, 64x64, 32x32
+
+
+@pytest.mark.parametrize("variant", Q8_TILES)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (17, 33, 64), (31, 65, 192), (64, 128, 320), (129, 130, 1088)])
+def test_q8_0_tiles(gpu, variant, M, N, K):
+    # Edges of the tiles in M and N, and numbers of block pairs that leave k groups without one (K = 64
+    # to 320 over four groups). f32 sums of exact products: the gate of the other Q8_0 tests.
+    from test_gpu_q8_0 import make_weights, q8_gpu
+    p = gpu.Plan()
+    p.family, p.variant = 8, variant
+    blocks, _, _ = make_weights(N, K, 40 + variant)
+    Xh = O.f16_bits(O.normal(M * K, 41 + M, 0.0, 1.0)).reshape(M, K)
+    assert frob(q8_gpu(gpu, Xh, blocks, N, plan=p), O.q8_0_gemm(Xh, blocks, N)) <= 1e-5
+
+
+@pytest.mark.parametrize("variant", Q8_TILES)
+def test_q8_0_tiles_keep_infinities(gpu, variant):
+    # An infinite activation in the last block pair of the last row: that row's outputs are +-inf (a
+    # k group without a pair of its own must add nothing), the others finite.
+    from test_gpu_q8_0 import make_weights, q8_gpu
+    M, N, K = 33, 40, 192
+    p = gpu.Plan()
+    p.family, p.variant = 8, variant
+    blocks, q, _ = make_weights(N, K, 3)
+    X = O.normal(M * K, 4, 0.0, 1.0).reshape(M, K)
+    X[M - 1, K - 1] = np.inf
+    y = q8_gpu(gpu, O.f16_bits(X), blocks, N, plan=p)
+    sign = np.asarray(q).reshape(N, K)[:, K - 1]
+    assert np.array_equal(y[M - 1][sign != 0], np.where(sign[sign != 0] > 0, np.inf, -np.inf).astype(np.float32))
+    assert np.isfinite(y[:M - 1]).all()

@@ -390,6 +390,15 @@ constexpr double kActBytesPerUsPerCu = 100e3;  // activation bytes per us per CU
 // row family's 2 us figure, which covers a cold start, overstates it here).
 constexpr double kQ8LatencyUs = 1.0;
 
+// A launch of `wgs` workgroups of `iters` k rounds each for more than 16 activation rows.
+double q8_many_us(const Hcs& h, const Q8Many& v, int64_t wgs, int64_t iters, int resident) {
+  const double work = v.work / mfma_clock_scale(h);
+  const int64_t slots = int64_t(cus(h)) * resident;
+  const int64_t full = wgs / slots, rest = wgs % slots;
+  const double last = rest ? std::max(v.lat_us, double((rest + cus(h) - 1) / cus(h)) * work) : 0.0;
+  return v.fixed_us + (double(iters) + v.tail) * (double(full) * std::max(v.lat_us, resident * work) + last);
+}
+
 std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
   const Workload w = workload_of(t);
   std::vector<Cand> cs;
@@ -492,7 +501,10 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     const double narrow_us = double(w.bytes) / (double(std::min<int64_t>(grid, cus(h))) * cu_share);
     const double stream =
         std::max(stream_us(h, double(w.bytes), grid, resident, inflight, false, 0.0, kQ8LatencyUs), narrow_us);
-    const double cost = launch_us(h) + stream + issue_us + gen_us + act_us + rounds_us + hide_us;
+    double cost = launch_us(h) + stream + issue_us + gen_us + act_us + rounds_us + hide_us;
+    if (s.M > 16)  // every 16 rows stream and convert the weights again
+      cost = std::max(launch_us(h) + stream,
+                      q8_many_us(h, v.many, grid, rounds, std::max(1, std::min<int>(16 / v.waves, int(lds_cu(h) / lds)))));
     Cand c;
     c.plan.family = Family::Q8Gemm;
     c.plan.variant = i;
@@ -506,6 +518,30 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
                  " resident per CU";
     c.cost = cost;
     cs.push_back(c);
+  }
+  for (int i = 0; i < kNumQ8TileVariants && s.M > 16; ++i) {
+    const Q8TileVariant v = kQ8TileVariants[i];
+    char key[64];
+    std::snprintf(key, sizeof key, "q8_0:tile%dx%d,k%d", v.bm, v.bn, v.ks);
+    const int64_t lds = int64_t(2) * v.ks * ((v.bm + v.bn) * 128 + v.bn * 8);
+    if (lds > lds_block(h)) {
+      reject(log, std::string(key) + " violates LDS " + std::to_string(lds) + " <= " + std::to_string(lds_block(h)));
+      continue;
+    }
+    Cand c;
+    c.plan.family = Family::Q8Gemm;
+    c.plan.variant = kNumQ8Variants + i;
+    c.plan.tile_m = v.bm;
+    c.plan.tile_n = v.bn;
+    c.plan.tile_k = 64 * v.ks;
+    c.plan.threads = v.wm * v.wn * v.ks * 64;
+    c.plan.split_k = v.ks;
+    c.plan.grid = ((s.M + v.bm - 1) / v.bm) * ((s.N + v.bn - 1) / v.bn);
+    c.plan.key = key;
+    c.plan.why = std::to_string(c.plan.grid) + " tiles, weights converted once per " + std::to_string(v.bm) + " rows";
+    c.cost = std::max(launch_us(h) + double(w.bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
+                      q8_many_us(h, v.many, c.plan.grid, (npairs + v.ks - 1) / v.ks, v.resident));
+    cs.push_back(std::move(c));
   }
   return pick(cs, "q8_0", log, err);
 }

@@ -25,8 +25,9 @@
 // lane's outputs all belong to one weight row and its two block scales are one LDS broadcast.
 //
 // K must be a multiple of 64 (whole block pairs per row).
-// Two kernel forms: q8_0_gemm_kernel (MFMA tiles of 16 weight rows, any M) below, and
-// q8_0_gemv_kernel (M = 1: one weight row per wavefront on the vector ALUs) further down.
+// Three kernel forms: q8_0_gemm_kernel (MFMA tiles of 16 weight rows, any M) below, q8_0_gemv_kernel
+// (M = 1: one weight row per wavefront on the vector ALUs) and q8_0_tile_kernel (more than 16 rows)
+// further down.
 // Work split of q8_0_gemm_kernel: grid.x = groups of 16 NT weight rows, grid.y = 16-row groups of activations. With
 // NT > 1 each activation fragment (read from global memory per workgroup) feeds NT MFMA tiles of
 // weights: every workgroup reads all of its activation rows over K, so for M = 16 the activation
@@ -39,6 +40,9 @@
 #include "../launch.hpp"
 #include "../variants.hpp"
 #include "common.hpp"
+
+#include <type_traits>
+#include <utility>
 
 namespace uk::kern {
 
@@ -462,11 +466,272 @@ __global__ void __launch_bounds__(WAVES * 64)
   if (lane == 0 && n < N) Y[n] = y;
 }
 
+// ---------------------------------------------------------------------------------------
+// q8_0_tile_kernel: a BM x BN tile per workgroup for more than 16 activation rows. The kernels above
+// re-read and re-convert every weight for each 16 rows of activations (32 times at M = 512); here a
+// weight is converted to f16 once per BM rows, on its way into LDS. Step of k: one block pair (64 k)
+// per k group, operands staged through registers a whole round ahead as in gemm_any.hip. Each block's
+// 16x16x32 MFMA starts from zero and its four sums are scaled and added in f32 (X first: a lane's four
+// sums belong to one weight row, so it needs one scale), the same arithmetic as above.
+// Bound: per block and 16x16 tile the four multiply-adds take as long on the vector ALU as the MFMA on
+// the matrix cores, and the conversion comes on top; both share the time with LDS (half of the cycles
+// at 64x64) and the texture cache's tag lookups. 512x4096x4096: 85.4 -> 44.3 us (388 TFLOP/s),
+// 512x11008x4096 277 -> 126, 64x11008x4096 41.1 -> 22.4; up to 16 rows keep the kernels above. (Two k
+// groups in 64x64 tiles took 40 and 110 us, 128x128 tiles of one group 90 at 512x11008x4096, with
+// the sums of one chain; with as many chains as here they need more registers and are slower.)
+template <int BM, int BN, int WM, int WN, int S>
+struct Q8TileCfg {
+  static constexpr int kGroup = WM * WN * 64;  // threads of one k group
+  static constexpr int kThreads = kGroup * S;
+  static constexpr int kFM = BM / WM / 16, kFN = BN / WN / 16;
+  static constexpr int kNX = BM * 8 / kGroup;  // 16-byte activation chunks per thread and block pair
+  static constexpr int kNW = BN * 4 / kGroup;  // half blocks (16 quants) per thread and block pair
+  static constexpr int kSlot = (BM + BN) * 128 + BN * 8;
+  static constexpr int kPitch = BN / WN + 4;   // floats
+  static constexpr int kPipe = 2 * S * kSlot;
+  static constexpr int kRed = (S - 1) * BM * BN * 4;
+  static constexpr int kStage = WM * WN * (BM / WM) * kPitch * 4;
+  static constexpr int kLds = kPipe > kRed ? (kPipe > kStage ? kPipe : kStage) : (kRed > kStage ? kRed : kStage);
+};
+
+template <int BM, int BN, int WM, int WN, int S>
+__global__ void __launch_bounds__(WM* WN* S * 64)
+    q8_0_tile_kernel(const _Float16* __restrict__ X, const uint8_t* __restrict__ Wq, float* __restrict__ Y, int M, int N,
+                     int K, int tiles_m, int tiles_n) {
+  asm volatile("" ::"s"(X), "s"(Wq), "s"(Y), "s"(M), "s"(N), "s"(K), "s"(tiles_m), "s"(tiles_n));
+  using Cfg = Q8TileCfg<BM, BN, WM, WN, S>;
+  constexpr int FM = Cfg::kFM, FN = Cfg::kFN, NX = Cfg::kNX, NW = Cfg::kNW;
+  static_assert(NX >= 1 && NW >= 1, "every thread stages a share of both operands");
+  __shared__ __attribute__((aligned(1024))) char lds[Cfg::kLds];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kh = w / (WM * WN), wg = w % (WM * WN), wm = wg / WN, wn = wg % WN;
+  const int tg = tid - kh * Cfg::kGroup;
+
+  const int G = tiles_m * tiles_n;
+  const int xcd = blockIdx.x & 7, per = G >> 3, rem = G & 7;
+  const int lin = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  constexpr int kGroupM = 8;
+  const int per_group = kGroupM * tiles_n;
+  const int group = lin / per_group;
+  const int first_m = group * kGroupM;
+  const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
+  const int in_group = lin - group * per_group;
+  const int m0 = (first_m + in_group % gm) * BM, n0 = (in_group / gm) * BN;
+
+  const int npairs = K >> 6;
+  const int64_t row_bytes = (int64_t)npairs * 68;
+  // Staging lanes: activations as eight 16-byte chunks per row and pair; weights as four half blocks
+  // per row and pair (16 quants at byte 2 + 16 h of block b, 34 bytes apart). Rows past the edges
+  // read the last row (they feed only outputs that are not stored).
+  const int xrow = tg >> 3, xc = tg & 7;
+  const int wrow = tg >> 2, wb = (tg >> 1) & 1, wh = tg & 1;
+  // A pair is 17 dwords: d0 in the low half of dword 0, the even block's quants from byte 2, d1 in the
+  // high half of dword 8, the odd block's quants from dword 9. Each lane loads whole dwords: 16 bytes
+  // at dword 0, 4, 9 or 13 and the dword 4, 8, 8 or 13 that completes them (unaligned 16-byte loads
+  // of the quants and 2-byte loads of the scales kept the texture cache busy all the time: 95.7k tag
+  // lookups per CU in a launch of 98k cycles, 62k now).
+  const int wext = wb ? (wh ? 0 : -4) : 16;
+  const int wshift = wb ? 0 : 2;
+  const int p0 = kh < npairs ? kh : npairs - 1;
+  const _Float16* xp[NX];
+  const uint8_t* wp[NW];
+#pragma unroll
+  for (int u = 0; u < NX; ++u) {
+    const int r = m0 + u * (Cfg::kGroup / 8) + xrow;
+    xp[u] = X + (int64_t)(r < M ? r : M - 1) * K + p0 * 64 + xc * 8;
+  }
+#pragma unroll
+  for (int u = 0; u < NW; ++u) {
+    const int r = n0 + u * (Cfg::kGroup / 4) + wrow;
+    wp[u] = Wq + (int64_t)(r < N ? r : N - 1) * row_bytes + p0 * 68 + wb * 36 + wh * 16;
+  }
+  u32x4 rx[2][NX], rw[2][NW];
+  uint32_t rd[2][NW];
+  // Loads of round t into register set t % 2. Past the group's last pair they read that pair again
+  // (multiply skips it): no branch, so the compiler can wait for one round's loads by count while the
+  // next round's are in flight.
+  auto load = [&](auto set_c, int t) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    const int more = (t + 1) * S + kh < npairs;
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      rx[set][u] = *reinterpret_cast<const u32x4*>(xp[u]);
+      xp[u] += more * S * 64;
+    }
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      __builtin_memcpy(&rw[set][u], __builtin_assume_aligned(wp[u], 4), 16);
+      rd[set][u] = *reinterpret_cast<const uint32_t*>(wp[u] + wext);
+      wp[u] += more * S * 68;
+    }
+  };
+  auto store = [&](auto slot_c) __attribute__((always_inline)) {
+    constexpr int slot = decltype(slot_c)::value;
+    char* xs = lds + (slot * S + kh) * Cfg::kSlot;
+    char* ws = xs + BM * 128;
+    float* ds = reinterpret_cast<float*>(ws + BN * 128);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int r = u * (Cfg::kGroup / 8) + xrow;
+      *reinterpret_cast<u32x4*>(xs + r * 128 + ((xc ^ ((r >> 1) & 7)) << 4)) = rx[slot][u];
+    }
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      const int r = u * (Cfg::kGroup / 4) + wrow, c = 4 * wb + 2 * wh, f = (r >> 1) & 7;
+      const u32x4 v = rw[slot][u];
+      const uint32_t q0 = __builtin_amdgcn_alignbyte(v.y, v.x, wshift), q1 = __builtin_amdgcn_alignbyte(v.z, v.y, wshift);
+      const uint32_t q2 = __builtin_amdgcn_alignbyte(v.w, v.z, wshift);
+      const uint32_t q3 = __builtin_amdgcn_alignbyte(rd[slot][u], v.w, wshift);
+      *reinterpret_cast<f16x8*>(ws + r * 128 + ((c ^ f) << 4)) = q8_to_f16x8(q0, q1);
+      *reinterpret_cast<f16x8*>(ws + r * 128 + (((c + 1) ^ f) << 4)) = q8_to_f16x8(q2, q3);
+      if (wh == 0) ds[wb * BN + r] = half_bits_to_float(wb ? rd[slot][u] >> 16 : v.x);
+    }
+  };
+  const int fi = lane & 15, fg = lane >> 4;
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Even and odd blocks sum apart, so an output is eight chains over the four k groups, as many as the
+  // split-k kernels above have: two groups of one chain each rounded off 1.5 times as much against 64
+  // bits (512x4096x4096: 1.5e-7, 9.3e-8 now, 9.7e-8 there).
+  f32x4 acc[FM][FN], part[2][FM][FN];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) part[c][i][j] = zero;
+  auto multiply = [&](auto slot_c) __attribute__((always_inline)) {
+    constexpr int slot = decltype(slot_c)::value;
+    const char* xs = lds + (slot * S + kh) * Cfg::kSlot;
+    const char* ws = xs + BM * 128;
+    const float* ds = reinterpret_cast<const float*>(ws + BN * 128);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int c = ((4 * b + fg) ^ ((fi >> 1) & 7)) << 4;
+      f16x8 fx[FM], fw[FN];
+      float d[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        fx[i] = *reinterpret_cast<const f16x8*>(xs + (wm * (BM / WM) + i * 16 + fi) * 128 + c);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        fw[j] = *reinterpret_cast<const f16x8*>(ws + (wn * (BN / WN) + j * 16 + fi) * 128 + c);
+        d[j] = ds[b * BN + wn * (BN / WN) + j * 16 + fi];
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const f32x4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(fx[i], fw[j], zero, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) part[b][i][j][r] = fmaf(d[j], s[r], part[b][i][j][r]);
+        }
+    }
+  };
+
+  // Round t: its operands sit in slot t % 2; the next round's, loaded two rounds ago, go into the other
+  // slot (every wavefront passed the barrier after reading it), the loads of round t + 3 take their
+  // registers, and only then does it multiply. Slots and register sets are compile-time constants.
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  auto round = [&](auto slot_c, int t) __attribute__((always_inline)) {
+    std::integral_constant<int, decltype(slot_c)::value ^ 1> next;
+    store(next);
+    load(next, t + 3);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t * S + kh < npairs) multiply(slot_c);
+    lds_barrier();
+  };
+  load(I0{}, 0);
+  load(I1{}, 1);
+  store(I0{});
+  load(I0{}, 2);
+  lds_barrier();
+  for (int t = 0; t * S < npairs; t += 2) {
+    round(I0{}, t);
+    round(I1{}, t + 1);
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = part[0][i][j][r] + part[1][i][j][r];
+  if constexpr (S > 1) {
+    f32x4* red = reinterpret_cast<f32x4*>(lds);
+    if (kh > 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) red[(((kh - 1) * FM + i) * FN + j) * Cfg::kGroup + tg] = acc[i][j];
+    }
+    __syncthreads();
+    if (kh == 0) {
+#pragma unroll
+      for (int s = 0; s < S - 1; ++s)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const f32x4 p = red[((s * FM + i) * FN + j) * Cfg::kGroup + tg];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] += p[r];
+          }
+    }
+    __syncthreads();
+    if (kh > 0) return;
+  }
+  // A lane holds rows 4 g .. 4 g + 3 of one column: through LDS to whole rows.
+  float* stage = reinterpret_cast<float*>(lds) + wg * (BM / WM) * Cfg::kPitch;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) stage[(i * 16 + 4 * fg + r) * Cfg::kPitch + j * 16 + fi] = acc[i][j][r];
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  constexpr int kRowChunks = BN / WN / 4;
+  const int mw = m0 + wm * (BM / WM), nw = n0 + wn * (BN / WN);
+#pragma unroll 4
+  for (int id = lane; id < BM / WM * kRowChunks; id += 64) {
+    const int r = id / kRowChunks, q = id % kRowChunks;
+    const int m = mw + r, n = nw + q * 4;
+    if (m >= M || n >= N) continue;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(stage + r * Cfg::kPitch + q * 4);
+    float* dst = Y + (int64_t)m * N + n;
+    if (N - n >= 4) {
+      __builtin_memcpy(dst, &v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < N - n) dst[e] = v[e];
+    }
+  }
+}
+
 }  // namespace uk::kern
 
 namespace uk {
 
 namespace {
+template <int... Is>
+hipError_t q8_tile_dispatch(int tile, const void* X, const void* Wq, float* Y, int64_t M, int64_t N, int64_t K,
+                            hipStream_t s, std::integer_sequence<int, Is...>) {
+  hipError_t e = hipErrorInvalidValue;
+  auto go = [&](auto i_c) {
+    constexpr Q8TileVariant v = kQ8TileVariants[decltype(i_c)::value];
+    const int64_t tm = (M + v.bm - 1) / v.bm, tn = (N + v.bn - 1) / v.bn;
+    constexpr int threads = v.wm * v.wn * v.ks * 64;
+    if (tm * tn * threads > UINT32_MAX) return;  // one grid dimension's limit in work items
+    hipLaunchKernelGGL((kern::q8_0_tile_kernel<v.bm, v.bn, v.wm, v.wn, v.ks>), dim3((unsigned)(tm * tn)), dim3(threads),
+                       0, s, static_cast<const _Float16*>(X), static_cast<const uint8_t*>(Wq), Y, (int)M, (int)N, (int)K,
+                       (int)tm, (int)tn);
+    e = hipGetLastError();
+  };
+  (void)((Is == tile && (go(std::integral_constant<int, Is>{}), true)) || ...);
+  return e;
+}
+
 template <int WAVES>
 hipError_t q8_gemv_go(const void* X, const void* Wq, float* Y, int64_t N, int64_t K, hipStream_t s) {
   const dim3 grid((unsigned)((N + WAVES - 1) / WAVES));
@@ -527,7 +792,8 @@ hipError_t q8_go(const void* X, const void* Wq, float* Y, int64_t M, int64_t N, 
 
 hipError_t launch_q8_gemm(const Plan& p, const void* X, const void* Wq, float* Y, int64_t M, int64_t N, int64_t K,
                           hipStream_t s) {
-  if (p.family != Family::Q8Gemm || p.variant < 0 || p.variant >= kNumQ8Variants) return hipErrorInvalidValue;
+  if (p.family != Family::Q8Gemm || p.variant < 0 || p.variant >= kNumQ8Variants + kNumQ8TileVariants)
+    return hipErrorInvalidValue;
   // Whole block pairs per row keep every row (34*K/32 bytes) and pair 4-byte aligned.
   if (M <= 0 || N <= 0 || K <= 0 || K % 64) return hipErrorInvalidValue;
   // Row byte offsets are 64-bit, element indices 32-bit; grid limits.
@@ -537,6 +803,9 @@ hipError_t launch_q8_gemm(const Plan& p, const void* X, const void* Wq, float* Y
   // Activation rows are read as 16-byte vectors at 2*(m*K + 64p + 8g [+ 32]) bytes (16-byte
   // aligned when X is); the weight stream is copied as dwords (4-byte aligned rows and pairs).
   if ((((uintptr_t)X) & 15) || (((uintptr_t)Wq) & 3) || (((uintptr_t)Y) & 3)) return hipErrorInvalidValue;
+  if (p.variant >= kNumQ8Variants)
+    return q8_tile_dispatch(p.variant - kNumQ8Variants, X, Wq, Y, M, N, K, s,
+                            std::make_integer_sequence<int, kNumQ8TileVariants>{});
   const Q8Variant v = kQ8Variants[p.variant];
   if (v.gemv) {
     // One activation row; rows of whole block-pair quadruples (16-byte aligned), one pair per lane.

@@ -151,13 +151,37 @@ constexpr int gemm_skinny_nt_waves(int waves) { return 2 * waves <= 16 ? 2 * wav
 // share each activation fragment.
 // gemv: the M = 1 kernel instead (one weight row per wavefront, vector-ALU dot products, `waves`
 // rows per workgroup sharing the activation row in LDS, one block pair per lane: K <= 4096).
+// many: more than 16 activation rows, where a workgroup's compute sets the time: fixed_us +
+// (rounds of k + tail) * sum over rounds of workgroups of max(lat_us, n * work), n the workgroups a
+// CU holds (the form of kGemmAnyVariants' cost), fitted over 170 shapes of M 17-512, N 64-11008, K
+// 64-11008 together with the tile kernels' (below): the pick is 2% over the fastest on average.
+struct Q8Many {
+  double lat_us, work, fixed_us, tail;
+};
 struct Q8Variant {
   int waves, pairs, vec, db, nt, gemv;
+  Q8Many many;
 };
-constexpr Q8Variant kQ8Variants[] = {{16, 4, 4, 0, 1}, {16, 4, 1, 0, 1}, {8, 8, 4, 0, 1}, {8, 4, 1, 0, 1},
-                                     {8, 4, 4, 1, 1},  {4, 4, 4, 1, 1},  {4, 8, 4, 1, 1}, {8, 4, 4, 0, 4},
-                                     {8, 4, 4, 0, 1},  {8, 4, 4, 0, 3},  {4, 1, 4, 0, 1, 1}};
+constexpr Q8Variant kQ8Variants[] = {
+    {16, 4, 4, 0, 1, 0, {0.600, 3.633, 1.427, 0.000}}, {16, 4, 1, 0, 1, 0, {3.894, 0.000, 0.893, 0.260}},
+    {8, 8, 4, 0, 1, 0, {0.600, 3.102, 2.961, 0.000}},  {8, 4, 1, 0, 1, 0, {0.600, 1.999, 2.706, 0.000}},
+    {8, 4, 4, 1, 1, 0, {0.600, 1.826, 2.657, 0.000}},  {4, 4, 4, 1, 1, 0, {1.354, 1.016, 2.460, 0.000}},
+    {4, 8, 4, 1, 1, 0, {0.600, 2.249, 3.102, 0.000}},  {8, 4, 4, 0, 4, 0, {0.600, 4.217, 0.000, 0.365}},
+    {8, 4, 4, 0, 1, 0, {0.600, 1.846, 1.948, 0.000}},  {8, 4, 4, 0, 3, 0, {0.600, 3.443, 0.000, 0.455}},
+    {4, 1, 4, 0, 1, 1, {}}};
 constexpr int kNumQ8Variants = sizeof(kQ8Variants) / sizeof(kQ8Variants[0]);
+// Q8_0 GEMM tiles for more than 16 activation rows (q8_0_tile_kernel): bm x bn outputs per workgroup,
+// wm x wn wavefronts per k group, ks k groups. The plan's variant number is kNumQ8Variants + index.
+struct Q8TileVariant {
+  int bm, bn, wm, wn, ks, resident;
+  Q8Many many;
+};
+constexpr Q8TileVariant kQ8TileVariants[] = {
+    {32, 64, 1, 4, 4, 1, {0.730, 0.510, 0.000, 5.206}},
+    {64, 64, 2, 2, 4, 1, {0.930, 0.300, 0.000, 4.433}},
+    {32, 32, 1, 2, 4, 2, {0.509, 0.470, 2.264, 1.818}},
+};
+constexpr int kNumQ8TileVariants = sizeof(kQ8TileVariants) / sizeof(kQ8TileVariants[0]);
 
 // Implicit-GEMM conv on f32 MFMA (v_mfma_f32_32x32x2f32). Wide kernel (tile_strips 0): a
 // wavefront owns 32 output pixels x 64 output channels, `waves` wavefronts per workgroup, and
