@@ -547,6 +547,8 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
 }
 
 // ---------------------------------------------------------------------------------------
+constexpr double kConvGatherFactor = 1.6, kConvGatherFixedUs = 2.5;
+
 std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
   const double peak = h.peak_f32_mfma_tflops > 0 ? h.peak_f32_mfma_tflops : h.flops_gflops * 1e-3 / 16;
   const double clk = clock_ghz(h) * 1e3;  // clocks per microsecond
@@ -652,8 +654,12 @@ std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, S
     // waves / SIMDs wavefronts and sets the time.
     const int64_t wg_per_cu = (wgs + cus(h) - 1) / cus(h);
     const double waves_per_simd = std::ceil(double(wg_per_cu) * v.waves / simds(h));
-    const double cost =
-        launch_us(h) + waves_per_simd * tiles_per_wave * tile_cycles / (clk * v.eff * mfma_clock_scale(h));
+    // The gathering kernels' efficiencies were calibrated at one NCHW shape with 64 channels; over 220
+    // drawn shapes they take 1.55 times what those give (median) and at least 2.5 us more than the launch
+    // overhead, and conv_any is faster at each of 8 us or more.
+    const double cost = launch_us(h) + (ldsk ? 0.0 : kConvGatherFixedUs) +
+                        (ldsk ? 1.0 : kConvGatherFactor) * waves_per_simd * tiles_per_wave * tile_cycles /
+                            (clk * v.eff * mfma_clock_scale(h));
     Cand c;
     c.plan.family = Family::ConvIgemm;
     c.plan.variant = i;
@@ -668,6 +674,44 @@ std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, S
                  fmt("%.2f", v.eff);
     c.cost = cost;
     cs.push_back(c);
+  }
+  const bool nchw = t.layout == Layout::NCHW;
+  const bool vec = !nchw && s.Ci % 4 == 0 && s.pad == 0;
+  for (int i = 0; i < kNumConvAnyVariants; ++i) {
+    const ConvAnyVariant v = kConvAnyVariants[i];
+    char key[64];
+    std::snprintf(key, sizeof key, "conv_any:%dx%d,k%d", v.bm, v.bn, v.ks);
+    if (!conv_any_supported(nchw, s.Nb, s.Ci, s.H, s.W, s.Co, s.Kh, s.Kw, s.Ho, s.Wo)) {
+      reject(log, std::string(key) + " violates taps<=49, 32-bit image offsets, k*inner<2^32");
+      continue;
+    }
+    if (int64_t(2) * v.ks * (v.bm + v.bn) * 128 + taps * v.bn * 4 > lds_block(h)) {
+      reject(log, std::string(key) + " violates LDS per workgroup");
+      continue;
+    }
+    const int64_t wgs = s.Nb * ((s.Co + v.bm - 1) / v.bm) * ((s.Ho * s.Wo + v.bn - 1) / v.bn);
+    const int64_t steps = (s.Ci * taps + 32 * v.ks - 1) / (32 * v.ks);
+    const double fit_scale = 157.2864 / 256.0 / (peak * mfma_clock_scale(h) / double(cus(h)));
+    const double work = (nchw ? v.work_nchw : vec ? v.work_vec : v.work_hwc) * fit_scale;
+    const double lat = vec ? v.lat_vec_us : v.lat_us;
+    const int64_t slots = int64_t(cus(h)) * v.resident;
+    const int64_t full = wgs / slots, rest = wgs % slots;
+    const double last = rest ? std::max(lat, double((rest + cus(h) - 1) / cus(h)) * work) : 0.0;
+    Cand c;
+    c.plan.family = Family::ConvIgemm;
+    c.plan.variant = kNumConvVariants + i;
+    c.plan.tile_m = v.bm;
+    c.plan.tile_n = v.bn;
+    c.plan.tile_k = 32 * v.ks;
+    c.plan.threads = v.wm * v.wn * v.ks * 64;
+    c.plan.split_k = v.ks;
+    c.plan.grid = wgs;
+    c.plan.key = key;
+    c.plan.why = std::to_string(wgs) + " tiles of " + std::to_string(v.bm) + " channels x " + std::to_string(v.bn) +
+                 " pixels, input gathered once per tile into LDS";
+    c.cost = std::max(launch_us(h) + double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
+                      v.fixed_us + (double(steps) + v.tail) * (double(full) * std::max(lat, v.resident * work) + last));
+    cs.push_back(std::move(c));
   }
   return pick(cs, "conv", log, err);
 }

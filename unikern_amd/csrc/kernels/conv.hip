@@ -950,7 +950,9 @@ hipError_t conv_tile_dispatch(bool nchw, int taps, const kern::ConvArgs& a, int6
 
 hipError_t launch_conv_igemm(const Plan& p, const Shape& sh, Layout lay, const float* X, const float* Wt,
                              const float* scale, float* Y, hipStream_t s) {
-  if (p.family != Family::ConvIgemm || p.variant < 0 || p.variant >= kNumConvVariants) return hipErrorInvalidValue;
+  if (p.family != Family::ConvIgemm || p.variant < 0 || p.variant >= kNumConvVariants + kNumConvAnyVariants)
+    return hipErrorInvalidValue;
+  if (p.variant >= kNumConvVariants) return launch_conv_any(p.variant - kNumConvVariants, sh, lay, X, Wt, scale, Y, s);
   const ConvVariant v = kConvVariants[p.variant];
   const bool nchw = lay == Layout::NCHW;
   if (!nchw && lay != Layout::NT) return hipErrorInvalidValue;

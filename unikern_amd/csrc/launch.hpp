@@ -34,6 +34,8 @@ hipError_t launch_q8_gemm(const Plan& p, const void* X, const void* Wq, float* Y
 // wavefronts per workgroup.
 constexpr int probe_mfmas_per_iter(int form) { return form == 16 ? 8 : 4; }
 hipError_t launch_mfma_probe(int form, int workgroups, int iters, unsigned long long* out, hipStream_t s);
+hipError_t launch_conv_any(int variant, const Shape& sh, Layout lay, const float* X, const float* Wt, const float* scale,
+                           float* Y, hipStream_t s);
 hipError_t launch_conv_igemm(const Plan& p, const Shape& sh, Layout lay, const float* X, const float* Wt,
                              const float* scale, float* Y, hipStream_t s);
 

@@ -268,6 +268,32 @@ inline bool conv_l16_supported(bool nchw, long kh, long kw, long stride, long pa
          16 * (g.gp + 4) < kConvL16IndexLimit && N * g.wpi < kConvL16IndexLimit;
 }
 
+// Implicit-GEMM conv of any kernel size, stride, padding and channel count (conv_any_kernel): bm output
+// channels x bn pixels of one image per workgroup, wm x wn wavefronts per k group, ks k groups. The
+// plan's variant number is kNumConvVariants + index. Cost: fixed_us + (32 ks-deep steps of k + tail) *
+// sum over rounds of max(lat, n * work), n the workgroups a CU holds (the form of kGemmAnyVariants'
+// cost), fitted over 220 drawn shapes (7-256 pixels a side, 3-256 channels, kernels of 1, 3 and 5): the
+// pick is 1.2% over the fastest on average. work: NCHW, HWC with C a multiple of 4 (16-byte loads), HWC.
+struct ConvAnyVariant {
+  int bm, bn, wm, wn, ks, resident;
+  double lat_us, lat_vec_us, work_nchw, work_vec, work_hwc, fixed_us, tail;
+};
+constexpr ConvAnyVariant kConvAnyVariants[] = {
+    {64, 64, 2, 2, 1, 3, 1.198, 0.692, 0.957, 0.630, 1.097, 2.843, 0.832},
+    {64, 64, 2, 2, 2, 2, 0.800, 0.500, 1.987, 1.294, 2.203, 2.689, 0.453},
+    {32, 64, 1, 4, 2, 2, 0.800, 0.500, 1.425, 0.772, 1.684, 2.823, 0.312},
+    {32, 64, 2, 2, 1, 4, 0.901, 0.426, 0.671, 0.384, 0.930, 3.175, 0.561},
+};
+constexpr int kNumConvAnyVariants = sizeof(kConvAnyVariants) / sizeof(kConvAnyVariants[0]);
+// Byte offsets within one image's X are 32-bit, k and pixel indices 31-bit, and the quotient k / inner by
+// mulhi is exact for k * inner < 2^32.
+inline bool conv_any_supported(bool nchw, long N, long C, long H, long W, long Oc, long kh, long kw, long Ho, long Wo) {
+  const long taps = kh * kw, K = C * taps, inner = nchw ? taps : C;
+  if (N <= 0 || C <= 0 || Oc <= 0 || Ho <= 0 || Wo <= 0 || taps <= 0 || taps > 49) return false;
+  if ((nchw ? H * W : H * W * C) * 4 > 0x7fffffffL || Ho * Wo > 0x3fffffffL) return false;
+  return K < 0x1000000L && K * inner < 0xffffffffL;
+}
+
 // Sustained shader clock (GHz) of the matrix-core probe (uk_probe_mfma: one wavefront per SIMD
 // issuing only v_mfma_f32_16x16x32_f16 on switching random operands, its primary form) on the
 // parts where the GEMM and conv efficiencies above were fitted (2.01-2.03 GHz measured; the same

@@ -31,8 +31,8 @@ KERNELS = {
     "gemm_f16": re.compile(r"gemm_f16_(tn|pp|w4|w4s|w4k|w4k16)_kernel"),
     "gemm_f32": re.compile(r"gemm_f32_kernel"),
     "gemm_generic": re.compile(r"gemm_any_kernel|gemm_skinny_(tn|nt)_kernel"),
-    "conv": re.compile(r"conv_igemm_kernel|conv_tile_kernel|conv_lds_kernel|conv_lds16_kernel"),
-    "q8_0": re.compile(r"q8_0_gemm_kernel|q8_0_gemv_kernel"),
+    "conv": re.compile(r"conv_igemm_kernel|conv_tile_kernel|conv_lds_kernel|conv_lds16_kernel|conv_any_kernel"),
+    "q8_0": re.compile(r"q8_0_gemm_kernel|q8_0_gemv_kernel|q8_0_tile_kernel"),
 }
 COPY_BYTES_READ = 4096 * 4096 * 4 + 4096 * 4
 COPY_BYTES_WRITTEN = 4096 * 4096 * 4
