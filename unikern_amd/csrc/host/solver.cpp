@@ -185,16 +185,22 @@ std::optional<Plan> solve_rows(const Hcs& h, const KmlTree& t, const Shape& s, S
     cs.push_back(c);
   }
   if (!cs.empty()) return pick(cs, "rows", log, err);
-  // Fallback for any row length: stream the row.
+  // Any other row length: the row in registers through unaligned loads, or streamed when it is longer.
   Plan p;
   p.family = Family::RowsStream;
-  p.threads = kRowsStreamThreads;
-  p.grid = s.L;
-  const int passes = t.op == OpKind::Softmax ? 3 : (t.op == OpKind::RmsNorm ? 2 : 1);
-  p.predicted_us = launch_us(h) + double(s.L * s.C * 4) * passes / (hbm_gbps(h) * 1e3) + double(s.L * s.C * 4) / (hbm_gbps(h) * 1e3);
+  const int pick = rows_any_pick(s.L, s.C);
+  if (pick >= 0) {
+    p.tpr = kRowsAny[pick].tpr;
+    p.vec = kRowsAny[pick].nv;
+  }
+  p.threads = pick >= 0 ? std::max(p.tpr, 256) : kRowsStreamThreads;
+  p.grid = pick >= 0 ? (s.L * p.tpr + p.threads - 1) / p.threads : s.L;
+  const int passes = pick >= 0 ? 1 : (t.op == OpKind::Softmax ? 3 : (t.op == OpKind::RmsNorm ? 2 : 1));
+  const double pass_us = double(s.L * s.C * 4) / (hbm_gbps(h) * 1e3 * (pick >= 0 ? kStreamEff : 1.0));
+  p.predicted_us = launch_us(h) + pass_us * passes + (t.op == OpKind::Reduction ? 0.0 : pass_us);
   p.feasible = 1;
   p.key = "rows_stream";
-  p.why = "row length not register-resident; streamed";
+  p.why = pick >= 0 ? "row of any length in registers, unaligned loads" : "row length not register-resident; streamed";
   return p;
 }
 

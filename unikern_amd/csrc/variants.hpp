@@ -55,6 +55,27 @@ constexpr int kNumRowsVariants = sizeof(kRowsVariants) / sizeof(kRowsVariants[0]
 inline bool channelscale_rows_form(long L, long C) { return C % 4 == 0 && C > 2048 && C <= 4096 && L <= 0x7fffffffL; }
 constexpr int kRowsStreamThreads = 256;
 
+// Rows of any length that the variants above do not hold (C not a multiple of 4, or longer):
+// rows_any_kernel keeps the row in registers, tpr threads with nv unaligned float4 each. The entry is
+// the smallest that holds the row (rows_any_pick); few rows take the widest teams, because a CU holds
+// one row at a time then and its loads all go out at once.
+struct RowsAnyVariant {
+  int tpr, nv;
+};
+constexpr RowsAnyVariant kRowsAny[] = {{64, 1},   {64, 2},   {64, 3},   {64, 4},   {64, 6},    {64, 8},    {256, 3},
+                                       {256, 4},  {256, 5},  {256, 6},  {256, 8},  {256, 10},  {256, 12},  {256, 16},
+                                       {1024, 1}, {1024, 2}, {1024, 3}, {1024, 4}, {1024, 5},  {1024, 6},  {1024, 8},
+                                       {1024, 10}, {1024, 12}, {1024, 15}, {1024, 18}};
+constexpr int kNumRowsAny = sizeof(kRowsAny) / sizeof(kRowsAny[0]);
+constexpr long kRowsAnyFew = 512;  // rows up to which 1024 threads take a row of more than 2048 floats
+inline int rows_any_pick(long L, long C) {
+  for (int i = 0; i < kNumRowsAny; ++i) {
+    if (kRowsAny[i].tpr == 256 && L <= kRowsAnyFew) continue;
+    if (C <= long(kRowsAny[i].tpr) * kRowsAny[i].nv * 4) return i;
+  }
+  return -1;  // longer rows are streamed
+}
+
 // 1-D reduce: pass-1 partial count and threads.
 constexpr int kReduceParts = 2048;
 constexpr int kReduceThreads = 256;
