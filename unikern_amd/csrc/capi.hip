@@ -202,7 +202,7 @@ constexpr size_t kStaticScratchBytes = size_t(1) << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 size_t scratch_bytes(const KmlTree& t) {
-  return t.op == OpKind::Reduction && t.ndims == 1 ? sizeof(float) * kReduceParts : 0;
+  return t.op == OpKind::Reduction && t.ndims == 1 && shape_of(t).C > kReduceOneMax ? sizeof(float) * kReduceParts : 0;
 }
 
 // uk_launch's scratch: the 1-D reduce's pass-1 partials in a file-scope device array of their
@@ -325,7 +325,7 @@ int dispatch(const KmlTree& t, const Plan& p, const void* const* in, void* out, 
       break;
     case OpKind::Reduction:
       if (t.ndims == 1) {
-        if (!ws.ptr || ws.bytes < scratch_bytes(t))
+        if (const size_t need = scratch_bytes(t); need && (!ws.ptr || ws.bytes < need))
           return fail(UK_HIP_FAILURE, "UNIKERN_ERROR what=scratch reason=no partials buffer for the 1-D reduce");
         e = launch_reduce1d(static_cast<const float*>(in[0]), static_cast<float*>(ws.ptr), static_cast<float*>(out),
                             s.C, st);

@@ -555,6 +555,9 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
 // ---------------------------------------------------------------------------------------
 constexpr double kConvGatherFactor = 1.6, kConvGatherFixedUs = 2.5;
 
+// One pass of 65536 floats by the 1-D reduce's single workgroup.
+constexpr double kReduceOnePassUs = 1.5;
+
 std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
   const double peak = h.peak_f32_mfma_tflops > 0 ? h.peak_f32_mfma_tflops : h.flops_gflops * 1e-3 / 16;
   const double clk = clock_ghz(h) * 1e3;  // clocks per microsecond
@@ -844,10 +847,18 @@ std::optional<Plan> solve(const Hcs& h, const KmlTree& t, SolveLog* log, std::st
       if (t.ndims == 1) {
         Plan p;
         p.family = Family::Reduce1D;
+        p.feasible = 1;
+        if (s.C <= kReduceOneMax) {
+          p.threads = kReduceOneThreads;
+          p.grid = 1;
+          p.predicted_us = launch_us(h) + kReduceOnePassUs * std::ceil(double(s.C) / 65536.0);
+          p.key = "reduce1d:one";
+          p.why = "one workgroup, one launch";
+          return p;
+        }
         p.threads = kReduceThreads;
         p.grid = kReduceParts;
         p.predicted_us = 2 * launch_us(h) + double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3);
-        p.feasible = 1;
         p.key = "reduce1d:parts=" + std::to_string(kReduceParts);
         p.why = "two deterministic passes (partials, one-workgroup fold)";
         return p;

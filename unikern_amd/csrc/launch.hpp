@@ -15,6 +15,7 @@ enum class RowOp : int { Sum = 0, RmsNorm = 1, Softmax = 2 };
 hipError_t launch_rows(const Plan& p, RowOp op, const float* X, const float* W, float* Y, int64_t L, int64_t C,
                        float eps, hipStream_t s);
 hipError_t launch_channelscale(const float* X, const float* S, float* Y, int64_t L, int64_t C, hipStream_t s);
+// partials: kReduceParts floats; not used where n <= kReduceOneMax.
 hipError_t launch_reduce1d(const float* X, float* partials, float* Y, int64_t n, hipStream_t s);
 
 hipError_t launch_gemm_f16(const Plan& p, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,

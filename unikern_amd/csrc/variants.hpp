@@ -76,9 +76,14 @@ inline int rows_any_pick(long L, long C) {
   return -1;  // longer rows are streamed
 }
 
-// 1-D reduce: pass-1 partial count and threads.
+// 1-D reduce: pass-1 partial count and threads of the two-pass form, and the length up to which one
+// workgroup sums the vector in one launch instead: that takes 4.1 us up to 65536 floats and 1.5 us per
+// 65536 more until 262144 (8.8 us; the CU's cache no longer serves it beyond, 17.3 us at 400001), the two
+// launches ordered by an event 9.0-10.2 us whatever the length up to 4 Mi floats.
 constexpr int kReduceParts = 2048;
 constexpr int kReduceThreads = 256;
+constexpr int kReduceOneThreads = 1024;
+constexpr long kReduceOneMax = 1L << 18;
 
 // f16 MFMA GEMM, layout TN (A[M][K], B stored [N][K]).
 // bm x bn x bk macro tile; wm x wn waves; stages of LDS buffering; swz selects the LDS
