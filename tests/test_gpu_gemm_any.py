@@ -120,3 +120,14 @@ def test_q8_0_tiles_keep_infinities(gpu, variant):
     sign = np.asarray(q).reshape(N, K)[:, K - 1]
     assert np.array_equal(y[M - 1][sign != 0], np.where(sign[sign != 0] > 0, np.inf, -np.inf).astype(np.float32))
     assert np.isfinite(y[:M - 1]).all()
+
+
+@pytest.mark.parametrize("M, N, K", [(1, 1, 1), (255, 191, 63), (256, 192, 64), (257, 193, 65), (513, 385, 321), (130, 960, 72)])
+def test_256x192(gpu, M, N, K):
+    # Variant 11, compiled for B [N][K] only: the edges of its tile, and columns of no power of two.
+    A, B = f16_inputs(M, N, K, 930 + N, tn=True)
+    got = O.f16_to_f32(run(gpu, A, B, "fp16", "TN", 11, off=N % 4))
+    assert frob(got, O.gemm_f16q(A, B, True)) <= 1e-3
+    if M == 257:
+        with pytest.raises(gpu.UnikernError):
+            run(gpu, A, B.reshape(K, N), "fp16", "NT", 11, off=0)

@@ -326,7 +326,7 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
   cs.reserve(cs.size() + kNumGemmAnyVariants);
   for (const GemmAnyVariant& entry : kGemmAnyVariants) {
     const GemmAnyVariant& v = entry.id == 0 && s.M <= 64 && s.N <= 64 ? gemm_any_variant(7) : entry;
-    if (v.f16_only && !f16) continue;
+    if ((v.f16_only && !f16) || (!tn && v.nt_factor == 0)) continue;
     const int64_t slab = f16 ? 64 : 32;  // k of one 128-byte row segment
     char key[64];
     int64_t wgs, iters, lds;

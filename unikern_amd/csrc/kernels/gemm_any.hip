@@ -24,8 +24,8 @@
 //   steps' loads in flight. Bound by the stream of B.
 //
 // Measured against the bounds-checked 64x64x16 kernel these replaced (element loads, two barriers per
-// 16 k), one box, inputs rotating over three sets: f16 TN 1000x11008x4096 2667 -> 106.7 us (846
-// TFLOP/s; 256x256), 16x11008x4096 251 -> 23.9 us (3.8 TB/s; skinny), f16 NT 512x9728x2560 440 ->
+// 16 k), one box, inputs rotating over three sets: f16 TN 1000x11008x4096 2667 -> 96.8 us (932
+// TFLOP/s; 256x192), 16x11008x4096 251 -> 23.9 us (3.8 TB/s; skinny), f16 NT 512x9728x2560 440 ->
 // 47.0 us (543 TFLOP/s; 256x128), f32 NT 1000^3 131 -> 24.8 us (81 TFLOP/s; 64x64 in two k groups),
 // and against 64 bits the f32 sums are no further off (4.0e-7 against 5.7e-7).
 #include "../launch.hpp"
@@ -538,7 +538,7 @@ dim3 any_grid(int64_t wgs) {
   return wgs <= kRow ? dim3((unsigned)wgs) : dim3((unsigned)kRow, (unsigned)((wgs + kRow - 1) / kRow));
 }
 
-constexpr int kGemmAnyNarrow = 7;  // the skinny 16x32 entry
+constexpr int kGemmAnyNarrow = 8;  // the skinny 16x32 entry
 static_assert(kGemmAnyVariants[kGemmAnyNarrow].id == 8 && kGemmAnyVariants[kGemmAnyNarrow].mt == 1, "a skinny variant");
 
 template <int I, typename T>
@@ -553,8 +553,12 @@ hipError_t any_go(bool bt, const T* a, const T* b, T* c, int64_t M, int64_t N, i
     const int64_t tm = (M + v.bm - 1) / v.bm, tn = (N + v.bn - 1) / v.bn;
     if (tm * tn > INT32_MAX) return hipErrorInvalidValue;
     constexpr int D = v.bm * v.bn >= 128 * 64 ? 1 : 2;  // registers for two load sets
-    auto* k = bt ? kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, true>
-                 : kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, false>;
+    auto* k = kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, true>;
+    if constexpr (v.nt_factor > 0) {
+      if (!bt) k = kern::gemm_any_kernel<T, v.bm, v.bn, v.wm, v.wn, v.ks, D, false>;
+    } else {
+      if (!bt) return hipErrorInvalidValue;
+    }
     hipLaunchKernelGGL(k, any_grid(tm * tn), dim3(Cfg::kThreads), 0, s, a, b, c, (int)M, (int)N, (int)K, (int)tm,
                        (int)tn);
     return hipGetLastError();

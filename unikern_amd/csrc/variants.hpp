@@ -143,6 +143,12 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // sum says, no variant has sustained more than kGemmAnyPeakF16 / F32 of the matrix-core peak.
 // The 64x64 variant 0 is the one any plan falls back to; a single tile of it (M, N <= 64) runs as
 // variant 7, whose 16-column workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
+// nt_factor 0: not compiled for B [K][N].
+// Variant 11 (256x192, TN only) is for products whose 256x256 tiles leave a quarter of the CUs idle or
+// spill into a new round: 1000x11008x4096 (232 tiles for 172) 107 -> 97 us, 1454x5888x1408 43 -> 37,
+// 3637x2887x3584 98 -> 86; picked at five of 49 drawn TN shapes and the fastest at each. For B [K][N] its
+// three chunks per thread do not split into pairs of k, and the 128x192 tile that would, in two k groups,
+// gained 1% at best over 256x128 there (46.5 against 46.8 us at 512x9728x2560): not compiled.
 // id: the plan's variant number (1 is gemm_f32_kernel). resident: workgroups per CU by LDS and registers.
 struct GemmAnyVariant {
   int id, bm, bn, wm, wn, ks, mt, nt, waves, unroll, resident, f16_only;
@@ -155,6 +161,7 @@ constexpr GemmAnyVariant kGemmAnyVariants[] = {
     {4, 128, 64, 2, 2, 1, 0, 0, 0, 0, 3, 0, 0.662, 0.473, 1.183, 1.020, 2.908, 0.854, 1.099},
     {5, 256, 128, 4, 2, 1, 0, 0, 0, 0, 1, 1, 0.600, 0.926, 0.000, 1.096, 0.000, 4.178, 1.156},
     {6, 256, 256, 2, 4, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.573, 0.000, 1.089, 0.000, 3.277, 1.138},
+    {11, 256, 192, 2, 4, 1, 0, 0, 0, 0, 1, 1, 0.600, 1.280, 0.000, 0.000, 0.000, 5.214, 1.221},
     {7, 16, 16, 0, 0, 0, 1, 1, 8, 4, 2, 0, 0.720, 0.766, 0.794, 2.324, 1.485, 0.000, 1.147},
     {8, 16, 32, 0, 0, 0, 1, 2, 4, 4, 4, 0, 0.608, 0.596, 0.649, 1.443, 1.606, 0.500, 1.237},
     {9, 32, 32, 0, 0, 0, 2, 2, 8, 2, 2, 0, 0.600, 1.473, 1.933, 1.493, 0.951, 0.230, 1.171},
