@@ -878,9 +878,9 @@ std::optional<Plan> solve(const Hcs& h, const KmlTree& t, SolveLog* log, std::st
         p.key = "channelscale:rows";
         p.why = "one wavefront per row, S in LDS, grouped stores";
       } else {
-        p.grid = std::min<int64_t>((s.L * s.C / 4 + 255) / 256, 256 * 32);
-        p.key = "channelscale:grid_stride";
-        p.why = "elementwise float4 grid-stride";
+        p.grid = channelscale_grid(s.L * s.C);
+        p.key = "channelscale:flat";
+        p.why = "16-byte accesses over the flat array, any row length";
       }
       return p;
     }

@@ -53,6 +53,14 @@ constexpr int kNumRowsVariants = sizeof(kRowsVariants) / sizeof(kRowsVariants[0]
 // Standalone channelscale in the grouped-store row form (one wavefront per row of at most 4096
 // floats, more than half of its lanes busy); other shapes take the float4 grid-stride kernel.
 inline bool channelscale_rows_form(long L, long C) { return C % 4 == 0 && C > 2048 && C <= 4096 && L <= 0x7fffffffL; }
+// Other shapes go as a flat array (channelscale_flat_kernel): workgroups of 4096 floats, or of 1024 where
+// there would be fewer than two of those per CU. Rows of 2049-4096 floats in multiples of 4 keep the row
+// form (4096 x 4096: 21.4 us; 4096 x 4097, flat, 24.8).
+constexpr long kChannelScaleSmall = 512L * 4096;
+inline long channelscale_grid(long n) {
+  const long per = n <= kChannelScaleSmall ? 1024 : 4096;
+  return (n + per - 1) / per;
+}
 constexpr int kRowsStreamThreads = 256;
 
 // Rows of any length that the variants above do not hold (C not a multiple of 4, or longer):
