@@ -23,14 +23,14 @@ SHAPES = [(1, 1, 1), (1, 3, 2), (5, 7, 3), (16, 64, 64), (17, 65, 63), (63, 33, 
           (257, 260, 1091)]
 
 
-def run(uk, A, B, dtype, layout, variant, off):
+def run(uk, A, B, dtype, layout, variant, off, family=6):
     """One launch with every operand `off` elements past a 256-byte boundary."""
     M, K = A.shape
     N = B.shape[0] if layout == "TN" else B.shape[1]
     es = A.itemsize
     d = uk.make_desc("gemm", [M, N, K], dtype=dtype, layout=layout)
     p = uk.Plan()
-    p.family, p.variant = 6, variant
+    p.family, p.variant = family, variant
     guard = 64
     bufs = []
     for a in (A, B):
@@ -131,3 +131,23 @@ def test_256x192(gpu, M, N, K):
     if M == 257:
         with pytest.raises(gpu.UnikernError):
             run(gpu, A, B.reshape(K, N), "fp16", "NT", 11, off=0)
+
+
+@pytest.mark.parametrize("dtype, layout, M, N, K", [("fp32", "TN", 64, 64, 64), ("fp32", "NT", 64, 192, 64), ("fp32", "NT", 128, 960, 128),
+                                                    ("fp32", "TN", 64, 1984, 512), ("fp16", "TN", 128, 128, 32),
+                                                    ("fp16", "TN", 128, 640, 1024), ("fp16", "TN", 128, 1664, 96)])
+def test_few_whole_tiles_take_any_element_alignment(gpu, dtype, layout, M, N, K):
+    # The solver's own plan, whichever kernel it names, at shapes of whole tiles too few for the aligned kernels.
+    plan = gpu.solve(gpu.make_desc("gemm", [M, N, K], dtype=dtype, layout=layout)).plan
+    if dtype == "fp16":
+        A, B = f16_inputs(M, N, K, 950, tn=True)
+        R = O.gemm_f16q(A, B, True)
+    else:
+        A = O.uniform(M * K, 951, -1.0, 1.0).reshape(M, K)
+        B = O.uniform(N * K, 952, -1.0, 1.0).reshape((N, K) if layout == "TN" else (K, N))
+        R = O.gemm_f32(A, B, layout == "TN")
+    for off in (0, 1):
+        got = run(gpu, A, B, dtype, layout, plan.variant, off, plan.family)
+        if dtype == "fp16":
+            got = O.f16_to_f32(got)
+        assert frob(got, R) <= (1e-3 if dtype == "fp16" else 1e-5)

@@ -149,7 +149,7 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // over 515 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every variant measured at each, both
 // types and layouts): the pick's time is about 2% over the fastest variant's on average. Whatever the
 // sum says, no variant has sustained more than kGemmAnyPeakF16 / F32 of the matrix-core peak.
-// The 64x64 variant 0 is the one any plan falls back to; a single tile of it (M, N <= 64) runs as
+// The 64x64 variant 0 is the one any plan falls back to; a product of a single tile of it (M, N <= 64) runs as
 // variant 7, whose 16-column workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
 // nt_factor 0: not compiled for B [K][N].
 // Variant 11 (256x192, TN only) is for products whose 256x256 tiles leave a quarter of the CUs idle or
