@@ -590,16 +590,26 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   };
   const int fi = lane & 15, fg = lane >> 4;
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Even and odd blocks sum apart, so an output is eight chains over the four k groups, as many as the
-  // split-k kernels above have: two groups of one chain each rounded off 1.5 times as much against 64
-  // bits (512x4096x4096: 1.5e-7, 9.3e-8 now, 9.7e-8 there).
-  f32x4 acc[FM][FN], part[2][FM][FN];
+  // Summation in blocks: `part` runs over the eight blocks of four rounds, then goes into `acc`. Its
+  // roundings grow with half the chain, those of `acc` with a sixteenth of a k group's length, so the sum
+  // rounds off less than the split-k kernels' at any K: one chain per wavefront there (8 or 16 chains),
+  // and one fused multiply-add per block in both (a sum of even and a sum of odd blocks, as many registers,
+  // cost a short K one more rounding: 4.6e-8 against 4.1e-8 at K = 64).
+  f32x4 acc[FM][FN], part[FM][FN];
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = part[i][j] = zero;
+  auto fold = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) part[c][i][j] = zero;
+      for (int j = 0; j < FN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += part[i][j][r];
+        part[i][j] = zero;
+      }
+  };
   auto multiply = [&](auto slot_c) __attribute__((always_inline)) {
     constexpr int slot = decltype(slot_c)::value;
     const char* xs = lds + (slot * S + kh) * Cfg::kSlot;
@@ -624,7 +634,7 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
         for (int j = 0; j < FN; ++j) {
           const f32x4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(fx[i], fw[j], zero, 0, 0, 0);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) part[b][i][j][r] = fmaf(d[j], s[r], part[b][i][j][r]);
+          for (int r = 0; r < 4; ++r) part[i][j][r] = fmaf(d[j], s[r], part[i][j][r]);
         }
     }
   };
@@ -650,13 +660,9 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   for (int t = 0; t * S < npairs; t += 2) {
     round(I0{}, t);
     round(I1{}, t + 1);
+    if (t & 2) fold();
   }
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = part[0][i][j][r] + part[1][i][j][r];
+  fold();
   if constexpr (S > 1) {
     f32x4* red = reinterpret_cast<f32x4*>(lds);
     if (kh > 0) {
