@@ -2,7 +2,8 @@
 
 An output is a sum of K/32 scaled blocks in f32. The split-k kernels sum one chain per wavefront; the
 tiles sum in blocks of eight, which rounds off less at any K. So the sixteen-wavefront kernel
-(variant 1, any K) bounds the tiles' error against binary64 over the same inputs.
+(variant 1, any K) bounds the tiles' error against binary64 over the same inputs, and the solver takes
+no split-k kernel of fewer, longer chains in its place.
 """
 import numpy as np
 import pytest
@@ -30,3 +31,17 @@ def test_tiles_round_off_no_more_than_sixteen_chains(gpu, K):
             assert np.array_equal(ys[v].view(np.uint32), ys[1].view(np.uint32))
         # 30720 outputs: the ratio of two such 2-norms scatters by 1 / sqrt(2 * 30720) = 0.4%.
         assert frob(ys[v], r) <= 1.01 * frob(ys[1], r), v
+
+
+@pytest.mark.parametrize("M,N,K", [(72, 64, 9536), (132, 563, 9792), (256, 67, 8320), (34, 175, 9856), (106, 508, 10752),
+                                   (259, 64, 9664), (128, 384, 8768)])
+def test_solver_keeps_sixteen_chains(uk, M, N, K):
+    # Shapes whose cheapest split-k kernel by the weight stream has sixteen wavefronts: a kernel of
+    # fewer takes longer and rounds off more.
+    s = uk.solve(uk.make_desc("gemm", [M, N, K], dtype="q8_0", layout="TN"))
+    assert s.key.startswith("q8_0:tile") or s.plan.split_k == 16
+
+
+def test_solver_keeps_the_streams_kernel_over_several_rounds(uk):
+    s = uk.solve(uk.make_desc("gemm", [375, 250, 10752], dtype="q8_0", layout="TN"))
+    assert s.key == "q8_0:waves=8,pairs=4,vec=4,nt=3"

@@ -396,6 +396,10 @@ constexpr double kActBytesPerUsPerCu = 100e3;  // activation bytes per us per CU
 // row family's 2 us figure, which covers a cold start, overstates it here).
 constexpr double kQ8LatencyUs = 1.0;
 
+// Tiles are taken only where they are cheaper by more than the fits agree on (359x320x4352: 11.8 against
+// 11.9 us predicted, 12.7 against 11.1 measured).
+constexpr double kQ8TileMargin = 1.03;
+
 // A launch of `wgs` workgroups of `iters` k rounds each for more than 16 activation rows.
 double q8_many_us(const Hcs& h, const Q8Many& v, int64_t wgs, int64_t iters, int resident) {
   const double work = v.work / mfma_clock_scale(h);
@@ -405,9 +409,48 @@ double q8_many_us(const Hcs& h, const Q8Many& v, int64_t wgs, int64_t iters, int
   return v.fixed_us + (double(iters) + v.tail) * (double(full) * std::max(v.lat_us, resident * work) + last);
 }
 
+// More than 16 rows: which of the split-k kernels stand beside the tiles. A wavefront of theirs sums its
+// blocks of all rounds in one chain, so a variant is not offered if its chain is longer than that of the
+// variant the weight stream's cost ranks first: eight wavefronts for its sixteen beyond K = 2048 round off
+// 10-13% more against 64 bits and are 3-9% slower (72x64x9536: 14.8 against 13.5 us). With chains no longer,
+// the costs fitted below decide against the tiles, but not between split-k kernels of several rounds (375x250x10752:
+// the one they rank first 27.3, the stream's 22.2 us) nor for fewer wavefronts at one round (they are 1.3 us
+// high for sixteen there: 5.8 against 4.5 us measured at K <= 2048): there the stream's first takes the cost.
+void keep_q8_chains(std::vector<Cand>* cs, const std::vector<double>& stream_cost, int64_t npairs, SolveLog* log) {
+  size_t first = 0;
+  for (size_t i = 1; i < cs->size(); ++i)
+    if (stream_cost[i] < stream_cost[first] ||
+        (stream_cost[i] == stream_cost[first] && (*cs)[i].plan.key < (*cs)[first].plan.key))
+      first = i;
+  const auto chain = [&](const Cand& c) {
+    const Q8Variant& v = kQ8Variants[c.plan.variant];
+    return (npairs + v.waves * v.pairs - 1) / (v.waves * v.pairs) * v.pairs;
+  };
+  const int64_t longest = chain((*cs)[first]);
+  const int waves = (*cs)[first].plan.split_k;
+  const bool rounds = npairs > waves * kQ8Variants[(*cs)[first].plan.variant].pairs;
+  double cost = (*cs)[first].cost;
+  std::vector<Cand> kept;
+  for (size_t i = 0; i < cs->size(); ++i) {
+    const Cand& c = (*cs)[i];
+    if (i == first) continue;
+    if (chain(c) > longest) {
+      reject(log, c.plan.key + " violates chain of blocks <= " + std::to_string(2 * longest));
+    } else if (rounds || c.plan.split_k < waves) {
+      cost = std::min(cost, c.cost);
+    } else {
+      kept.push_back(c);
+    }
+  }
+  kept.push_back((*cs)[first]);
+  kept.back().cost = cost;
+  *cs = std::move(kept);
+}
+
 std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
   const Workload w = workload_of(t);
   std::vector<Cand> cs;
+  std::vector<double> stream_cost;  // M > 16: of cs[i], by the weight stream (the cost that ranks up to 16 rows)
   const int64_t npairs = s.K / 64;
   for (int i = 0; i < kNumQ8Variants; ++i) {
     const Q8Variant v = kQ8Variants[i];
@@ -508,9 +551,11 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     const double stream =
         std::max(stream_us(h, double(w.bytes), grid, resident, inflight, false, 0.0, kQ8LatencyUs), narrow_us);
     double cost = launch_us(h) + stream + issue_us + gen_us + act_us + rounds_us + hide_us;
-    if (s.M > 16)  // every 16 rows stream and convert the weights again
+    if (s.M > 16) {  // every 16 rows stream and convert the weights again
+      stream_cost.push_back(cost);
       cost = std::max(launch_us(h) + stream,
                       q8_many_us(h, v.many, grid, rounds, std::max(1, std::min<int>(16 / v.waves, int(lds_cu(h) / lds)))));
+    }
     Cand c;
     c.plan.family = Family::Q8Gemm;
     c.plan.variant = i;
@@ -525,6 +570,7 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     c.cost = cost;
     cs.push_back(c);
   }
+  if (s.M > 16 && !cs.empty()) keep_q8_chains(&cs, stream_cost, npairs, log);
   for (int i = 0; i < kNumQ8TileVariants && s.M > 16; ++i) {
     const Q8TileVariant v = kQ8TileVariants[i];
     char key[64];
@@ -546,7 +592,7 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     c.plan.key = key;
     c.plan.why = std::to_string(c.plan.grid) + " tiles, weights converted once per " + std::to_string(v.bm) + " rows";
     c.cost = std::max(launch_us(h) + double(w.bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
-                      q8_many_us(h, v.many, c.plan.grid, (npairs + v.ks - 1) / v.ks, v.resident));
+                      kQ8TileMargin * q8_many_us(h, v.many, c.plan.grid, (npairs + v.ks - 1) / v.ks, v.resident));
     cs.push_back(std::move(c));
   }
   return pick(cs, "q8_0", log, err);
