@@ -11,9 +11,11 @@
 //
 // Semantics kept from the reference CPU loops: rmsnorm y = (x * rms) * W with
 // rms = 1/sqrt(sum(x^2)/C + eps) (correctly rounded divide and sqrt); softmax
-// y = exp(x - max) / sum(exp(x - max)), here as 2^((x - max) log2 e) * (1 / sum) on v_exp_f32
+// y = exp(x - max) / sum(exp(x - max)), in rows_kernel as 2^((x - max) log2 e) * (1 / sum) on v_exp_f32
 // (exp_sub below): within about 2e-6 of the reference wherever the 1e-5 relative gate can see an
-// element, and a fifth of the vector instructions of a libm exp and a divide per element.
+// element, and a fifth of the vector instructions of a libm exp and a divide per element; in
+// rows_any_kernel to an ulp (exp_sub_ulp and a corrected quotient), as in the libm form of
+// rows_stream_kernel.
 #include <math.h>
 
 #include <mutex>
@@ -50,6 +52,19 @@ __device__ __forceinline__ void st4(f32x4* p, f32x4 v) {
 // instructions, which did not hide behind the row stream.)
 constexpr float kLog2eF = 1.44269502f;  // log2(e) rounded to binary32
 __device__ __forceinline__ float exp_sub(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kLog2eF); }
+
+// e^(x - m) to about an ulp of the subtraction's result, as a libm expf: (x - m) log2 e = n + r with n an
+// integer and |r| <= 1/2, the product's rounding and the binary32 log2(e)'s kept in r by two fused
+// multiply-adds, and 2^n applied by an exponent add that reaches the denormals. Below -104 the result is 0
+// (under half the smallest denormal), which is also what -inf gives; NaN stays NaN.
+constexpr float kLog2eLoF = 1.92596303e-8f;  // log2(e) - kLog2eF
+__device__ __forceinline__ float exp_sub_ulp(float x, float m) {
+  const float d = x - m;
+  const float n = __builtin_rintf(d * kLog2eF);
+  const float r = __builtin_fmaf(d, kLog2eLoF, __builtin_fmaf(d, kLog2eF, -n));
+  const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(r), (int)n);
+  return d < -104.f ? 0.f : e;
+}
 
 // TPR threads own one row at a time and each keeps NV float4 of it in registers; a workgroup
 // walks RPB rows (RPB > 1: the next row's loads are issued before the current row's reduction,
@@ -257,9 +272,11 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
 // 16-byte loads and stores at 4-byte aligned addresses (rows of an odd length start anywhere; the
 // hardware takes them in one instruction and a wavefront touches nine lines instead of eight) and the
 // one lane that holds the row's last, partial float4 going element by element. Bound by HBM. It
-// replaces three scalar passes with libm exponentials and a divide per element: softmax 2048 x 5003
-// 28.2 -> 13.4 us (6.1 TB/s), 64 x 70001 181 -> 12.4, RMSNorm 4096 x 4097 42.1 -> 30.0, row-sum
-// 1000 x 9999 14.0 -> 7.3.
+// replaces three scalar passes with libm exponentials and a divide per element: RMSNorm 4096 x 4097
+// 42.1 -> 30.0 us, row-sum 1000 x 9999 14.0 -> 7.3, softmax 2048 x 5003 28.8 -> 14.4 and 64 x 70001 146 -> 15.0
+// (inputs that stay in the 256 MiB MALL), element by element no further from 64 bits (relative rms 8.4e-7
+// on both sides, which is x - max's rounding). The exponent and the quotient cost softmax 4-25% over
+// rows_kernel's (13.1 and 11.9 us, relative rms 1.2e-6 and denormals lost), a libm expf and a divide 12-60%.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 template <int TPR, int NV, int OP>
@@ -354,13 +371,18 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      v[i] = f32x4{exp_sub(v[i].x, m), exp_sub(v[i].y, m), exp_sub(v[i].z, m), exp_sub(v[i].w, m)};
+      v[i] = f32x4{exp_sub_ulp(v[i].x, m), exp_sub_ulp(v[i].y, m), exp_sub_ulp(v[i].z, m), exp_sub_ulp(v[i].w, m)};
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
     s = fold(wave_sum(s), red[1], add);
+    // v / s: a product with the reciprocal, corrected by its remainder.
     const float inv = 1.0f / s;
+    auto quotient = [&](float a) __attribute__((always_inline)) {
+      const float q = a * inv;
+      return __builtin_fmaf(__builtin_fmaf(-q, s, a), inv, q);
+    };
 #pragma unroll
-    for (int i = 0; i < NV; ++i) put(i, f32x4{v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv});
+    for (int i = 0; i < NV; ++i) put(i, f32x4{quotient(v[i].x), quotient(v[i].y), quotient(v[i].z), quotient(v[i].w)});
   }
 }
 
