@@ -38,6 +38,7 @@ struct ConvAnyArgs {
   int inner;               // k = outer * inner + rest: taps (NCHW) or C (HWC)
   unsigned magic;          // ceil(2^32 / inner): k / inner = mulhi(k, magic) (inner > 1)
   int tiles_m, tiles_n;    // tiles of output channels and of one image's pixels
+  int tiles;               // of all images
   int64_t xstep, ystep;    // floats of one image of X and Y
 };
 
@@ -71,7 +72,9 @@ __global__ void __launch_bounds__(WM* WN* S * 64, 4)
   const int tg = tid - kh * Cfg::kGroup;
 
   const int per_image = a.tiles_m * a.tiles_n;
-  const int image = blockIdx.x / per_image, in_image = blockIdx.x - image * per_image;
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  if (id >= a.tiles) return;
+  const int image = id / per_image, in_image = id - image * per_image;
   const int m0 = in_image % a.tiles_m * BM, n0 = in_image / a.tiles_m * BN;
   const float* const xb = a.x + image * a.xstep;
 
@@ -309,13 +312,13 @@ __global__ void __launch_bounds__(WM* WN* S * 64, 4)
 namespace uk {
 namespace {
 template <int MODE, int BM, int BN, int WM, int WN, int S, bool PAD>
-hipError_t conv_any_go(const kern::ConvAnyArgs& a, int64_t grid, hipStream_t s) {
+hipError_t conv_any_go(const kern::ConvAnyArgs& a, hipStream_t s) {
   using Cfg = kern::ConvAnyCfg<BM, BN, WM, WN, S>;
   static hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(&kern::conv_any_kernel<MODE, BM, BN, WM, WN, S, PAD>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, 163840);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((kern::conv_any_kernel<MODE, BM, BN, WM, WN, S, PAD>), dim3((unsigned)grid), dim3(Cfg::kThreads),
+  hipLaunchKernelGGL((kern::conv_any_kernel<MODE, BM, BN, WM, WN, S, PAD>), folded_grid(a.tiles), dim3(Cfg::kThreads),
                      Cfg::kMax + a.taps * BN * 4, s, a);
   return hipGetLastError();
 }
@@ -350,19 +353,20 @@ hipError_t launch_conv_any(int variant, const Shape& sh, Layout lay, const float
   a.xstep = sh.Ci * sh.H * sh.W;
   a.ystep = sh.Co * int64_t(a.P);
   const int64_t grid = sh.Nb * a.tiles_m * int64_t(a.tiles_n);
-  if (grid * v.wm * v.wn * v.ks * 64 > UINT32_MAX || grid > INT32_MAX) return hipErrorInvalidValue;
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  a.tiles = (int)grid;
   const bool pad = sh.pad != 0;
   const bool vec = !nchw && sh.Ci % 4 == 0 && !pad;
   hipError_t e = hipErrorInvalidValue;
   auto go = [&](auto i_c) {
     constexpr ConvAnyVariant c = kConvAnyVariants[decltype(i_c)::value];
     if (nchw)
-      e = pad ? conv_any_go<0, c.bm, c.bn, c.wm, c.wn, c.ks, true>(a, grid, s)
-              : conv_any_go<0, c.bm, c.bn, c.wm, c.wn, c.ks, false>(a, grid, s);
+      e = pad ? conv_any_go<0, c.bm, c.bn, c.wm, c.wn, c.ks, true>(a, s)
+              : conv_any_go<0, c.bm, c.bn, c.wm, c.wn, c.ks, false>(a, s);
     else if (vec)
-      e = conv_any_go<1, c.bm, c.bn, c.wm, c.wn, c.ks, false>(a, grid, s);
+      e = conv_any_go<1, c.bm, c.bn, c.wm, c.wn, c.ks, false>(a, s);
     else
-      e = conv_any_go<2, c.bm, c.bn, c.wm, c.wn, c.ks, true>(a, grid, s);
+      e = conv_any_go<2, c.bm, c.bn, c.wm, c.wn, c.ks, true>(a, s);
   };
   [&]<int... Is>(std::integer_sequence<int, Is...>) {
     (void)((Is == variant && (go(std::integral_constant<int, Is>{}), true)) || ...);

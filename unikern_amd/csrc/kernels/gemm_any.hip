@@ -532,12 +532,6 @@ __global__ void __launch_bounds__(W * 64)
 
 namespace uk {
 namespace {
-// Grids beyond one dimension's limit (2^32 work items) fold into y; the kernels flatten the id.
-dim3 any_grid(int64_t wgs) {
-  constexpr int64_t kRow = 1 << 20;
-  return wgs <= kRow ? dim3((unsigned)wgs) : dim3((unsigned)kRow, (unsigned)((wgs + kRow - 1) / kRow));
-}
-
 constexpr int kGemmAnyNarrow = 8;  // the skinny 16x32 entry
 static_assert(kGemmAnyVariants[kGemmAnyNarrow].id == 8 && kGemmAnyVariants[kGemmAnyNarrow].mt == 1, "a skinny variant");
 
@@ -559,7 +553,7 @@ hipError_t any_go(bool bt, const T* a, const T* b, T* c, int64_t M, int64_t N, i
     } else {
       if (!bt) return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(k, any_grid(tm * tn), dim3(Cfg::kThreads), 0, s, a, b, c, (int)M, (int)N, (int)K, (int)tm,
+    hipLaunchKernelGGL(k, folded_grid(tm * tn), dim3(Cfg::kThreads), 0, s, a, b, c, (int)M, (int)N, (int)K, (int)tm,
                        (int)tn);
     return hipGetLastError();
   } else {
@@ -568,10 +562,10 @@ hipError_t any_go(bool bt, const T* a, const T* b, T* c, int64_t M, int64_t N, i
     if (gm * gn > INT32_MAX) return hipErrorInvalidValue;
     constexpr int W2 = gemm_skinny_nt_waves(v.waves), U2 = v.unroll > 1 ? v.unroll / 2 : 1;
     if (bt)
-      hipLaunchKernelGGL((kern::gemm_skinny_tn_kernel<T, v.mt, v.nt, v.waves, v.unroll>), any_grid(gm * gn),
+      hipLaunchKernelGGL((kern::gemm_skinny_tn_kernel<T, v.mt, v.nt, v.waves, v.unroll>), folded_grid(gm * gn),
                          dim3(v.waves * 64), 0, s, a, b, c, (int)M, (int)N, (int)K, (int)gm, (int)gn);
     else
-      hipLaunchKernelGGL((kern::gemm_skinny_nt_kernel<T, v.mt, W2, U2>), any_grid(gm * gn), dim3(W2 * 64), 0, s, a, b,
+      hipLaunchKernelGGL((kern::gemm_skinny_nt_kernel<T, v.mt, W2, U2>), folded_grid(gm * gn), dim3(W2 * 64), 0, s, a, b,
                          c, (int)M, (int)N, (int)K, (int)gm, (int)gn);
     return hipGetLastError();
   }

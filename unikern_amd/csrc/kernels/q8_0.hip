@@ -509,8 +509,10 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   const int tg = tid - kh * Cfg::kGroup;
 
   const int G = tiles_m * tiles_n;
-  const int xcd = blockIdx.x & 7, per = G >> 3, rem = G & 7;
-  const int lin = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  if (id >= G) return;
+  const int xcd = id & 7, per = G >> 3, rem = G & 7;
+  const int lin = xcd * per + (xcd < rem ? xcd : rem) + (id >> 3);
   constexpr int kGroupM = 8;
   const int per_group = kGroupM * tiles_n;
   const int group = lin / per_group;
@@ -728,9 +730,9 @@ hipError_t q8_tile_dispatch(int tile, const void* X, const void* Wq, float* Y, i
     constexpr Q8TileVariant v = kQ8TileVariants[decltype(i_c)::value];
     const int64_t tm = (M + v.bm - 1) / v.bm, tn = (N + v.bn - 1) / v.bn;
     constexpr int threads = v.wm * v.wn * v.ks * 64;
-    if (tm * tn * threads > UINT32_MAX) return;  // one grid dimension's limit in work items
-    hipLaunchKernelGGL((kern::q8_0_tile_kernel<v.bm, v.bn, v.wm, v.wn, v.ks>), dim3((unsigned)(tm * tn)), dim3(threads),
-                       0, s, static_cast<const _Float16*>(X), static_cast<const uint8_t*>(Wq), Y, (int)M, (int)N, (int)K,
+    if (tm * tn > INT32_MAX) return;
+    hipLaunchKernelGGL((kern::q8_0_tile_kernel<v.bm, v.bn, v.wm, v.wn, v.ks>), folded_grid(tm * tn), dim3(threads), 0, s,
+                       static_cast<const _Float16*>(X), static_cast<const uint8_t*>(Wq), Y, (int)M, (int)N, (int)K,
                        (int)tm, (int)tn);
     e = hipGetLastError();
   };

@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
   constexpr int WPR = TPR / 64;
   __shared__ float red[2][WG / 64];
   const int tid = threadIdx.x, t = tid % TPR, wave = tid >> 6;
-  const int64_t row = (int64_t)blockIdx.x * (WG / TPR) + tid / TPR;
+  const int64_t row = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (WG / TPR) + tid / TPR;
   const bool active = row < L;  // rows past L are masked: every thread reaches every barrier
   const float* x = X + (active ? row : 0) * (int64_t)C;
   const int tail = C & 3, C4 = C >> 2;
@@ -444,7 +444,8 @@ __global__ void __launch_bounds__(256)
     channelscale_flat_kernel(const float* __restrict__ X, const float* __restrict__ S, float* __restrict__ Y, int64_t n,
                              unsigned C) {
   asm volatile("" ::"s"(X), "s"(S), "s"(Y), "s"(n), "s"(C));
-  const int64_t base = (int64_t)blockIdx.x * (U * 1024);
+  const int64_t base = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (U * 1024);
+  if (base >= n) return;
   const int64_t left = n - base;
   const int here = left < U * 1024 ? (int)left : U * 1024;
   const float* x = X + base;
@@ -629,7 +630,7 @@ hipError_t rows_any_dispatch(int pick, RowOp op, const float* X, const float* W,
     auto* k = op == RowOp::Sum       ? kern::rows_any_kernel<v.tpr, v.nv, 0>
               : op == RowOp::RmsNorm ? kern::rows_any_kernel<v.tpr, v.nv, 1>
                                      : kern::rows_any_kernel<v.tpr, v.nv, 2>;
-    hipLaunchKernelGGL(k, dim3((unsigned)((L + rows - 1) / rows)), dim3(wg), 0, s, X, W, Y, (int)L, (int)C, eps);
+    hipLaunchKernelGGL(k, folded_grid((L + rows - 1) / rows), dim3(wg), 0, s, X, W, Y, (int)L, (int)C, eps);
   };
   (void)((Is == pick && (go(std::integral_constant<int, Is>{}), true)) || ...);
   return hipGetLastError();
@@ -754,11 +755,11 @@ hipError_t launch_channelscale(const float* X, const float* S, float* Y, int64_t
   }
   const int64_t n = L * C;
   const int64_t grid = channelscale_grid(n);
-  if (grid * 256 > UINT32_MAX) return hipErrorInvalidValue;  // one grid dimension's limit in work items
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
   if (n <= kChannelScaleSmall)
-    hipLaunchKernelGGL(kern::channelscale_flat_kernel<1>, dim3((unsigned)grid), dim3(256), 0, s, X, S, Y, n, (unsigned)C);
+    hipLaunchKernelGGL(kern::channelscale_flat_kernel<1>, folded_grid(grid), dim3(256), 0, s, X, S, Y, n, (unsigned)C);
   else
-    hipLaunchKernelGGL(kern::channelscale_flat_kernel<4>, dim3((unsigned)grid), dim3(256), 0, s, X, S, Y, n, (unsigned)C);
+    hipLaunchKernelGGL(kern::channelscale_flat_kernel<4>, folded_grid(grid), dim3(256), 0, s, X, S, Y, n, (unsigned)C);
   return hipGetLastError();
 }
 

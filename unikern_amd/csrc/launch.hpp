@@ -10,6 +10,14 @@
 
 namespace uk {
 
+// The grid of `wgs` workgroups (at most 2^31 - 1): a grid dimension holds fewer than 2^32 work items, so more
+// than 2^20 workgroups fold into y. A kernel launched so flattens its id (blockIdx.y * gridDim.x +
+// blockIdx.x) and returns where that is past the last workgroup.
+inline dim3 folded_grid(int64_t wgs) {
+  constexpr int64_t kRow = 1 << 20;
+  return wgs <= kRow ? dim3((unsigned)wgs) : dim3((unsigned)kRow, (unsigned)((wgs + kRow - 1) / kRow));
+}
+
 enum class RowOp : int { Sum = 0, RmsNorm = 1, Softmax = 2 };
 
 hipError_t launch_rows(const Plan& p, RowOp op, const float* X, const float* W, float* Y, int64_t L, int64_t C,
