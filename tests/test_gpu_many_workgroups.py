@@ -90,3 +90,35 @@ def test_channelscale(gpu):
     for r in (0, L // 2, L - 1):
         assert np.array_equal(read(gpu, yb, r * n * 4, n), want)
     assert guard(gpu, yb, L * n * 4)
+
+
+def test_row_sums_of_multiples_of_four(gpu):
+    # Registers-resident rows of 64: 2^24 workgroups and one row more, in two launches.
+    L, n = (1 << 26) + 1, 64
+    xb, yb = gpu.DeviceBuffer(L * n * 4), output(gpu, L * 4)
+    xb.fill(0x3F)
+    gpu.launch(gpu.make_desc("reduce", [L, n]), [xb], yb)
+    want = 64 * np.full(1, 0x3F3F3F3F, np.uint32).view(np.float32)
+    assert (read(gpu, yb, 0, L) == want).all() and guard(gpu, yb, L * 4)
+
+
+def test_softmax_in_two_launches(gpu):
+    # Every element 1/64, in place of X; read back at the start, around the second launch's first row and at the end.
+    L, n = (1 << 26) + 1, 64
+    xb = output(gpu, L * n * 4)
+    xb.fill(0x3F)
+    gpu.launch(gpu.make_desc("softmax", [L, n]), [xb], xb)
+    for r in (0, (1 << 26) - 8, L - 1):
+        assert (read(gpu, xb, r * n * 4, n) == 1 / 64).all()
+
+
+def test_pixels_of_a_1x1_conv(gpu):
+    d = gpu.make_desc("conv", [16384, 16384, 1, 1, 1, 1], layout="NCHW", batch=4)
+    n = 4 << 28
+    xb, wb, yb = gpu.DeviceBuffer(n * 4), gpu.DeviceBuffer.from_array(np.float32([2])), output(gpu, n * 4)
+    xb.fill(0x3F)
+    gpu.launch(d, [xb, wb], yb)
+    want = 2 * np.full(1, 0x3F3F3F3F, np.uint32).view(np.float32)
+    for at in (0, n // 2, n - 4096):
+        assert (read(gpu, yb, at * 4, 4096) == want).all()
+    assert guard(gpu, yb, n * 4)

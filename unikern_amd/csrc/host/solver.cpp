@@ -297,6 +297,8 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
     const std::string key = "gemm_f32:64x64x64,w8";
     if (!(s.M % 64 == 0 && s.N % 64 == 0 && s.K % 64 == 0)) {
       reject(log, key + " violates M%64==0 && N%64==0 && K%64==0");
+    } else if (!grid_dim_holds((s.M / 64) * (s.N / 64), 512)) {
+      reject(log, key + " violates one grid dimension's work items");
     } else {
       // One 64x64 tile per workgroup, eight wavefronts (two per SIMD, splitting each k-tile):
       // the busiest CU's tiles at the calibrated fraction of its f32 MFMA rate.
@@ -472,6 +474,10 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
         continue;
       }
       const int64_t grid = (s.N + v.waves - 1) / v.waves;
+      if (!grid_dim_holds(grid, v.waves * 64)) {
+        reject(log, key + " violates one grid dimension's work items");
+        continue;
+      }
       const int resident =
           std::max(1, std::min<int>(waves_by_regs(h, 64) * simds(h) / v.waves, int(lds_cu(h) / lds)));
       const double inflight = double(v.waves) * double(npairs) * 68.0;
@@ -505,6 +511,10 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     }
     if (lds > lds_block(h)) {
       reject(log, key.str() + " violates LDS " + std::to_string(lds) + " <= " + std::to_string(lds_block(h)));
+      continue;
+    }
+    if (!grid_dim_holds((s.N + 16 * v.nt - 1) / (16 * v.nt), v.waves * 64)) {
+      reject(log, key.str() + " violates one grid dimension's work items");
       continue;
     }
     const int64_t per_round = int64_t(v.waves) * v.pairs;
@@ -636,6 +646,10 @@ std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, S
                        "index quotients below 2^21");
         continue;
       }
+      if (!grid_dim_holds(s.Nb * g.wpi, 512)) {
+        reject(log, k + " violates one grid dimension's work items");
+        continue;
+      }
       const int64_t wgs = s.Nb * g.wpi * ocb;
       const int64_t lds = 2 * (4 * kConvL16Rows * kConvL16Pitch + 9 * 4 * kConvL16WQuad) * 16;
       if (lds > lds_block(h)) {
@@ -703,6 +717,10 @@ std::optional<Plan> solve_conv(const Hcs& h, const KmlTree& t, const Shape& s, S
     }
     if (lds > lds_block(h)) {
       reject(log, key.str() + " violates LDS per workgroup");
+      continue;
+    }
+    if (!grid_dim_holds(wgs / oc_tiles, v.waves * 64)) {
+      reject(log, key.str() + " violates one grid dimension's work items");
       continue;
     }
     // Workgroups spread over the CUs; the busiest SIMD holds ceil(workgroups per CU) times

@@ -911,6 +911,7 @@ namespace {
 template <bool NCHW, int TAPS, int WAVES>
 hipError_t conv_go(const kern::ConvArgs& a, int64_t units, int oc_tiles, size_t lds, hipStream_t s) {
   const unsigned grid = (unsigned)((units + WAVES - 1) / WAVES);
+  if (!grid_dim_holds(grid, WAVES * 64)) return hipErrorInvalidValue;
   // Dynamic LDS above the default limit must be requested per kernel (once).
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&kern::conv_igemm_kernel<NCHW, TAPS, WAVES>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 163840);
@@ -933,6 +934,7 @@ namespace {
 template <bool NCHW, int TAPS, int S, int CB>
 hipError_t conv_tile_go(const kern::ConvArgs& a, int64_t units, int oc_tiles, hipStream_t s) {
   const unsigned grid = (unsigned)((units + S - 1) / S);
+  if (!grid_dim_holds(grid, S * 128)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((kern::conv_tile_kernel<NCHW, TAPS, S, CB>), dim3(grid, (unsigned)oc_tiles), dim3(S * 128), 0,
                      s, a);
   return hipGetLastError();
@@ -986,7 +988,7 @@ hipError_t launch_conv_igemm(const Plan& p, const Shape& sh, Layout lay, const f
     const ConvL16Geom g = conv_l16_geom(sh.Nb, sh.Ho, sh.Wo, (sh.Co + 63) / 64);
     const int64_t oc_blocks = (sh.Co + 63) / 64;
     // Input staging tasks (4 quads x rows x W / 4 columns) fit the 512 threads.
-    if (4 * kConvL16Rows * (sh.W / 4) > 512 || sh.Nb * g.wpi > INT32_MAX || oc_blocks > 65535)
+    if (4 * kConvL16Rows * (sh.W / 4) > 512 || !grid_dim_holds(sh.Nb * g.wpi, 512) || oc_blocks > 65535)
       return hipErrorInvalidValue;
     a.gp = (int)g.gp;
     a.wpi = (int)g.wpi;
@@ -1004,7 +1006,7 @@ hipError_t launch_conv_igemm(const Plan& p, const Shape& sh, Layout lay, const f
     if ((((uintptr_t)X) | ((uintptr_t)Wt)) & 15) return hipErrorInvalidValue;
     const int64_t tiles = (sh.Ho * sh.Wo + 64 * pt - 1) / (64 * pt);
     const int oc_tiles = (int)((sh.Co + 63) / 64);
-    if (sh.Nb * tiles > INT32_MAX || oc_tiles > 65535) return hipErrorInvalidValue;
+    if (!grid_dim_holds(sh.Nb * tiles, 256 * pt) || oc_tiles > 65535) return hipErrorInvalidValue;
     const dim3 grid((unsigned)(sh.Nb * tiles), (unsigned)oc_tiles);
     if (pt == 1) hipLaunchKernelGGL(kern::conv_lds_kernel<1>, grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL(kern::conv_lds_kernel<2>, grid, dim3(512), 0, s, a);

@@ -1547,7 +1547,7 @@ hipError_t launch_gemm_generic(int variant, DType dt, Layout lay, const void* A,
   auto b = static_cast<const float*>(B);
   auto c = static_cast<float*>(C);
   const int tm = int(M / 64), tn = int(N / 64);
-  if (int64_t(tm) * tn > INT32_MAX) return hipErrorInvalidValue;
+  if (!grid_dim_holds(int64_t(tm) * tn, 512)) return hipErrorInvalidValue;
   const dim3 g1((unsigned)(tm * tn));
   if (lay == Layout::TN)
     hipLaunchKernelGGL((kern::gemm_f32_kernel<true>), g1, dim3(512), 0, s, a, b, c, (int)M, (int)N, (int)K, tm, tn);

@@ -743,6 +743,7 @@ hipError_t q8_tile_dispatch(int tile, const void* X, const void* Wq, float* Y, i
 template <int WAVES>
 hipError_t q8_gemv_go(const void* X, const void* Wq, float* Y, int64_t N, int64_t K, hipStream_t s) {
   const dim3 grid((unsigned)((N + WAVES - 1) / WAVES));
+  if (!grid_dim_holds(grid.x, WAVES * 64)) return hipErrorInvalidValue;
   if (K == 4096)
     hipLaunchKernelGGL((kern::q8_0_gemv_kernel<WAVES, true>), grid, dim3(WAVES * 64), 0, s,
                        static_cast<const _Float16*>(X), static_cast<const uint8_t*>(Wq), Y, (int)N, (int)K);
@@ -761,6 +762,7 @@ constexpr int kQ8LdsLimit = 160 * 1024;
 template <int WAVES, int P, int VEC, bool DB, int NT>
 hipError_t q8_go(const void* X, const void* Wq, float* Y, int64_t M, int64_t N, int64_t K, hipStream_t s) {
   const dim3 grid((unsigned)((N + 16 * NT - 1) / (16 * NT)), (unsigned)((M + 15) / 16));
+  if (!grid_dim_holds(grid.x, WAVES * 64)) return hipErrorInvalidValue;
   // Activations through LDS at M <= 8 where the instantiation's LDS allows it.
   if constexpr (P == 4 && !DB) {
     if constexpr (q8_lds_bytes(WAVES, P, VEC, DB, NT, 1) <= kQ8LdsLimit) {

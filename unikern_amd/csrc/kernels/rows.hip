@@ -662,11 +662,19 @@ hipError_t rows_dispatch_op(RowOp op, const float* X, const float* W, float* Y, 
                             hipStream_t s) {
   constexpr int WG = TPR < 256 ? 256 : TPR;
   constexpr int RPW = WG / TPR;
-  const int64_t grid = (L + RPW * RPB - 1) / (RPW * RPB);
-  if constexpr (GS) {
-    if (C == int64_t(TPR) * NV * 4 && L % (RPW * RPB) == 0) return rows_go<TPR, NV, NT, RPB, GS, true>(op, X, W, Y, L, C, eps, grid, s);
+  // More rows than one grid dimension holds go in several launches.
+  constexpr int64_t kMost = kGridDimItems / WG * (RPW * RPB);
+  for (; L > 0; L -= kMost, X += kMost * C, Y += op == RowOp::Sum ? kMost : kMost * C) {
+    const int64_t n = L < kMost ? L : kMost;
+    const int64_t grid = (n + RPW * RPB - 1) / (RPW * RPB);
+    hipError_t e;
+    if (GS && C == int64_t(TPR) * NV * 4 && n % (RPW * RPB) == 0)
+      e = rows_go<TPR, NV, NT, RPB, GS, GS>(op, X, W, Y, n, C, eps, grid, s);
+    else
+      e = rows_go<TPR, NV, NT, RPB, GS, false>(op, X, W, Y, n, C, eps, grid, s);
+    if (e != hipSuccess) return e;
   }
-  return rows_go<TPR, NV, NT, RPB, GS, false>(op, X, W, Y, L, C, eps, grid, s);
+  return hipSuccess;
 }
 }  // namespace
 
@@ -675,9 +683,9 @@ hipError_t launch_rows(const Plan& p, RowOp op, const float* X, const float* W, 
   if (L <= 0 || C <= 0 || L > INT32_MAX || C > INT32_MAX) return hipErrorInvalidValue;
   if (op == RowOp::RmsNorm && !W) return hipErrorInvalidValue;
   if (p.family == Family::RowsStream) {
-    if (L > 0x7fffffff) return hipErrorInvalidValue;
     if (const int i = rows_any_pick(L, C); i >= 0)
       return rows_any_dispatch(i, op, X, W, Y, L, C, eps, s, std::make_integer_sequence<int, kNumRowsAny>{});
+    if (!grid_dim_holds(L, 256)) return hipErrorInvalidValue;  // 2^24 rows of more than 73728 floats: 4.9 TB
     switch (op) {
       case RowOp::Sum:
         hipLaunchKernelGGL(kern::rows_stream_kernel<0>, dim3((unsigned)L), dim3(256), 0, s, X, W, Y, (int)L, (int)C,

@@ -5,6 +5,11 @@
 
 namespace uk {
 
+// Work items of one grid dimension. The runtime takes a launch of more without an error and runs what is
+// left of the number modulo 2^32.
+constexpr long kGridDimItems = 0xffffffffL;
+inline bool grid_dim_holds(long workgroups, int threads) { return workgroups <= kGridDimItems / threads; }
+
 // Row family (row-sum, RMSNorm, softmax with the row held in registers).
 // tpr: threads per row (whole wavefronts), nv: float4 registers per thread.
 // A workgroup is max(tpr, 256) threads, i.e. 256/tpr rows per workgroup when tpr < 256.
