@@ -319,7 +319,7 @@ int dispatch(const KmlTree& t, const Plan& p, const void* const* in, void* out, 
         e = launch_q8_gemm(p, in[0], in[1], static_cast<float*>(out), s.M, s.N, s.K, st);
       else if ((p.family == Family::GemmF16 || p.variant == 1) &&
                ((((uintptr_t)in[0]) | ((uintptr_t)in[1]) | ((uintptr_t)out)) & 15) &&
-               gemm_few_tiles(t.dtype, t.layout, s.M, s.N, s.K))
+               gemm_few_tiles(t.dtype == DType::F16, t.layout == Layout::TN, s.M, s.N, s.K))
         e = launch_gemm_any(0, t.dtype, t.layout, in[0], in[1], out, s.M, s.N, s.K, st);
       else if (p.family == Family::GemmF16)
         e = launch_gemm_f16(p, in[0], in[1], out, s.M, s.N, s.K, st);

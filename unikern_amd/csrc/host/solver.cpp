@@ -386,8 +386,9 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
   }
   auto best = pick(cs, "gemm", log, err);
   if (best && best->family == Family::GemmGeneric && best->variant != 1)
-    best->why = std::to_string(best->grid) + " workgroups of " + std::to_string(best->threads) +
-                " threads, any shape, layout and element alignment";
+    best->why = std::to_string(best->grid) + " workgroups of " + std::to_string(best->threads) + " threads, any shape and layout, " +
+                (gemm_any_asks_alignment(best->variant, f16, tn, s.M, s.N, s.K) ? "16-byte aligned operands (many whole tiles)"
+                                                                               : "any element alignment");
   return best;
 }
 

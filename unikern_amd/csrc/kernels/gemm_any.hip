@@ -583,26 +583,13 @@ hipError_t any_dispatch(int variant, bool bt, const void* A, const void* B, void
 }
 }  // namespace
 
-static bool whole_tiles(DType dt, Layout lay, int64_t M, int64_t N, int64_t K) {
-  return dt == DType::F16 ? lay == Layout::TN && M % 128 == 0 && N % 128 == 0 && K % 32 == 0
-                          : M % 64 == 0 && N % 64 == 0 && K % 64 == 0;
-}
-
-bool gemm_few_tiles(DType dt, Layout lay, int64_t M, int64_t N, int64_t K) {
-  if (!whole_tiles(dt, lay, M, N, K)) return false;
-  return dt == DType::F16 ? (M / 128) * (N / 128) < 16 : (M / 64) * (N / 64) < 32;
-}
-
 hipError_t launch_gemm_any(int variant, DType dt, Layout lay, const void* A, const void* B, void* C, int64_t M, int64_t N,
                            int64_t K, hipStream_t s) {
   if (M <= 0 || N <= 0 || K <= 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return hipErrorInvalidValue;
   if (lay != Layout::NT && lay != Layout::TN) return hipErrorInvalidValue;
   if ((M + 63) / 64 > 65535) return hipErrorInvalidValue;
   const bool bt = lay == Layout::TN;
-  // Shapes of many whole tiles ask for 16-byte aligned operands whichever kernel the plan names (the
-  // direct-to-LDS kernels, which share these shapes, need it); the variant any plan falls back to and
-  // other shapes take any element alignment.
-  if (variant != 0 && whole_tiles(dt, lay, M, N, K) && !gemm_few_tiles(dt, lay, M, N, K) &&
+  if (gemm_any_asks_alignment(variant, dt == DType::F16, bt, M, N, K) &&
       ((((uintptr_t)A) | ((uintptr_t)B) | ((uintptr_t)C)) & 15))
     return hipErrorInvalidValue;
   constexpr auto seq = std::make_integer_sequence<int, kNumGemmAnyVariants>{};

@@ -34,9 +34,6 @@ hipError_t launch_gemm_generic(int variant, DType dt, Layout lay, const void* A,
                                int64_t N, int64_t K, hipStream_t s);
 hipError_t launch_gemm_any(int variant, DType dt, Layout lay, const void* A, const void* B, void* C, int64_t M, int64_t N,
                            int64_t K, hipStream_t s);
-// A GEMM of whole tiles with too few of them for the tile kernels that need 16-byte aligned operands
-// (fewer than 32 of 64x64 in f32, 16 of 128x128 in f16): it takes operands of any element alignment.
-bool gemm_few_tiles(DType dt, Layout lay, int64_t M, int64_t N, int64_t K);
 bool gemm_f32_tiled_supported(int64_t M, int64_t N, int64_t K);
 hipError_t launch_q8_gemm(const Plan& p, const void* X, const void* Wq, float* Y, int64_t M, int64_t N, int64_t K,
                           hipStream_t s);

@@ -187,6 +187,19 @@ constexpr const GemmAnyVariant& gemm_any_variant(int id) {
     if (v.id == id) return v;
   return kGemmAnyVariants[0];
 }
+// Products of many whole tiles (f16 TN: of 128x128x32; f32: of 64x64x64) ask for 16-byte aligned operands, whichever
+// kernel the plan names: the direct-to-LDS kernels, which share these shapes, need it, and whether a call is
+// taken must not hang on which of them a cost constant prefers. Few whole tiles (fewer than 16 or 32, which
+// those kernels rarely get), other shapes and variant 0 take any element alignment.
+inline bool gemm_whole_tiles(bool f16, bool tn, long M, long N, long K) {
+  return f16 ? tn && M % 128 == 0 && N % 128 == 0 && K % 32 == 0 : M % 64 == 0 && N % 64 == 0 && K % 64 == 0;
+}
+inline bool gemm_few_tiles(bool f16, bool tn, long M, long N, long K) {
+  return gemm_whole_tiles(f16, tn, M, N, K) && (f16 ? (M / 128) * (N / 128) < 16 : (M / 64) * (N / 64) < 32);
+}
+inline bool gemm_any_asks_alignment(int variant, bool f16, bool tn, long M, long N, long K) {
+  return variant != 0 && gemm_whole_tiles(f16, tn, M, N, K) && !gemm_few_tiles(f16, tn, M, N, K);
+}
 constexpr int gemm_skinny_nt_waves(int waves) { return 2 * waves <= 16 ? 2 * waves : 16; }
 
 // Q8_0 skinny GEMM: a workgroup owns 16 nt weight rows; each of its wavefronts copies `pairs`
