@@ -305,10 +305,6 @@ bool plan_matches(const KmlTree& t, const Plan& p) {
   return false;
 }
 
-// A single tile of the 64x64 GEMM variant runs as variant 7 (see kGemmAnyVariants). The shards of a
-// streamed GEMM follow the whole product's size, so that a short last shard sums in the same order.
-int gemm_one_tile_variant(int variant, const Shape& s) { return variant == 0 && s.M <= 64 && s.N <= 64 ? 7 : variant; }
-
 // Enqueue one launch of the op. Returns a uk_status.
 int dispatch(const KmlTree& t, const Plan& p, const void* const* in, void* out, hipStream_t st, const Scratch& ws) {
   const Shape s = shape_of(t);
@@ -324,8 +320,7 @@ int dispatch(const KmlTree& t, const Plan& p, const void* const* in, void* out, 
       else if (p.family == Family::GemmF16)
         e = launch_gemm_f16(p, in[0], in[1], out, s.M, s.N, s.K, st);
       else
-        e = launch_gemm_generic(p.shard_rows > 0 ? p.variant : gemm_one_tile_variant(p.variant, s), t.dtype, t.layout,
-                                in[0], in[1], out, s.M, s.N, s.K, st);
+        e = launch_gemm_generic(p.variant, t.dtype, t.layout, in[0], in[1], out, s.M, s.N, s.K, st);
       break;
     case OpKind::Conv:
       e = launch_conv_igemm(p, s, t.layout, static_cast<const float*>(in[0]), static_cast<const float*>(in[1]),
@@ -491,7 +486,6 @@ struct StreamGemm {
     M = sh.M;
     N = sh.N;
     K = sh.K;
-    if (p.family == Family::GemmGeneric) p.variant = gemm_one_tile_variant(p.variant, sh);
     es = t.dtype == DType::F16 ? 2 : 4;
     rows = std::min<int64_t>(p.shard_rows, M);
     if (rows <= 0) {

@@ -207,7 +207,8 @@ std::optional<Plan> solve_rows(const Hcs& h, const KmlTree& t, const Shape& s, S
 // ---------------------------------------------------------------------------------------
 constexpr double kGemmF32Eff = 0.72;  // gemm_f32_kernel's fraction of the f32 MFMA rate (calibrated at 1024^3)
 
-// The shortest time measured for any launch of kernels/gemm_any.hip.
+// About the shortest launch of kernels/gemm_any.hip (4.4 us on the part the costs were fitted on, 3.9 on the
+// quickest seen).
 constexpr double kGemmAnyFloorUs = 4.4;
 
 std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, SolveLog* log, std::string* err) {
@@ -326,8 +327,10 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
       launch_us(h) + std::max(double(workload_of(t).bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
                               flops / (peak_tflops * 1e6 * mfma_clock_scale(h) * (f16 ? kGemmAnyPeakF16 : kGemmAnyPeakF32)));
   cs.reserve(cs.size() + kNumGemmAnyVariants);
-  for (const GemmAnyVariant& entry : kGemmAnyVariants) {
-    const GemmAnyVariant& v = entry.id == 0 && s.M <= 64 && s.N <= 64 ? gemm_any_variant(7) : entry;
+  // A product of one 64x64 tile is offered variant 7 (64 KiB of LDS at most) instead of variant 0.
+  const bool one_tile = s.M <= 64 && s.N <= 64 && lds_block(h) >= 65536;
+  for (const GemmAnyVariant& v : kGemmAnyVariants) {
+    if (v.id == 0 && one_tile) continue;
     if ((v.f16_only && !f16) || (!tn && v.nt_factor == 0)) continue;
     const int64_t slab = f16 ? 64 : 32;  // k of one 128-byte row segment
     char key[64];
@@ -359,7 +362,7 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
       c.plan.split_k = waves;
     }
     // The kernel any shape falls back to is offered whatever the description says of LDS.
-    if (entry.id != 0 && lds > lds_block(h)) {
+    if (v.id != 0 && lds > lds_block(h)) {
       reject(log, std::string(key) + " violates LDS " + std::to_string(lds) + " <= " + std::to_string(lds_block(h)));
       continue;
     }
@@ -374,13 +377,13 @@ std::optional<Plan> solve_gemm(const Hcs& h, const KmlTree& t, const Shape& s, S
     // none beats the streaming rate of its operands or the matrix cores' sustained rate.
     c.cost = std::max({kGemmAnyFloorUs, rounds_us, roof_us});
     c.plan.family = Family::GemmGeneric;
-    c.plan.variant = entry.id;
+    c.plan.variant = v.id;
     c.plan.grid = wgs;
     c.plan.key = key;
-    if (entry.id == 0) {
-      c.plan.key = "gemm_generic:64x64x16";  // x16: k of one step of f32 fragments
-      c.plan.tile_m = c.plan.tile_n = 64;
-      c.plan.tile_k = 16;
+    if (v.id == 0) {
+      c.plan.key = "gemm_any:64x64,k1";  // first of several at the floor
+    } else if (v.id == 7 && one_tile) {
+      c.plan.key = "gemm_generic:64x64x16";  // the name a product of one 64x64 tile has always had
     }
     cs.push_back(std::move(c));
   }

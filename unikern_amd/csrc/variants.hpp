@@ -154,8 +154,8 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // over 515 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every variant measured at each, both
 // types and layouts): the pick's time is about 2% over the fastest variant's on average. Whatever the
 // sum says, no variant has sustained more than kGemmAnyPeakF16 / F32 of the matrix-core peak.
-// The 64x64 variant 0 is the one any plan falls back to; a product of a single tile of it (M, N <= 64) runs as
-// variant 7, whose 16-column workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
+// The 64x64 variant 0 is the one any shape falls back to; a product of a single tile of it (M, N <= 64) is offered
+// variant 7 in its place, whose 16-row workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
 // nt_factor 0: not compiled for B [K][N].
 // Variant 11 (256x192, TN only) is for products whose 256x256 tiles leave a quarter of the CUs idle or
 // spill into a new round: 1000x11008x4096 (232 tiles for 172) 107 -> 97 us, 1454x5888x1408 43 -> 37,
@@ -182,11 +182,6 @@ constexpr GemmAnyVariant kGemmAnyVariants[] = {
 };
 constexpr double kGemmAnyPeakF16 = 0.467, kGemmAnyPeakF32 = 0.80;
 constexpr int kNumGemmAnyVariants = sizeof(kGemmAnyVariants) / sizeof(kGemmAnyVariants[0]);
-constexpr const GemmAnyVariant& gemm_any_variant(int id) {
-  for (const GemmAnyVariant& v : kGemmAnyVariants)
-    if (v.id == id) return v;
-  return kGemmAnyVariants[0];
-}
 // Products of many whole tiles (f16 TN: of 128x128x32; f32: of 64x64x64) ask for 16-byte aligned operands, whichever
 // kernel the plan names: the direct-to-LDS kernels, which share these shapes, need it, and whether a call is
 // taken must not hang on which of them a cost constant prefers. Few whole tiles (fewer than 16 or 32, which
