@@ -199,7 +199,7 @@ std::optional<Plan> solve_rows(const Hcs& h, const KmlTree& t, const Shape& s, S
   const double pass_us = double(s.L * s.C * 4) / (hbm_gbps(h) * 1e3 * (pick >= 0 ? kStreamEff : 1.0));
   p.predicted_us = launch_us(h) + pass_us * passes + (t.op == OpKind::Reduction ? 0.0 : pass_us);
   p.feasible = 1;
-  p.key = "rows_stream";
+  p.key = pick >= 0 ? "rows_any:tpr=" + std::to_string(p.tpr) + ",nv=" + std::to_string(p.vec) : "rows_stream";
   p.why = pick >= 0 ? "row of any length in registers, unaligned loads" : "row length not register-resident; streamed";
   return p;
 }

@@ -683,7 +683,7 @@ hipError_t launch_rows(const Plan& p, RowOp op, const float* X, const float* W, 
   if (L <= 0 || C <= 0 || L > INT32_MAX || C > INT32_MAX) return hipErrorInvalidValue;
   if (op == RowOp::RmsNorm && !W) return hipErrorInvalidValue;
   if (p.family == Family::RowsStream) {
-    if (const int i = rows_any_pick(L, C); i >= 0)
+    if (const int i = rows_any_entry(p.tpr, p.vec, L, C); i >= 0)
       return rows_any_dispatch(i, op, X, W, Y, L, C, eps, s, std::make_integer_sequence<int, kNumRowsAny>{});
     if (!grid_dim_holds(L, 256)) return hipErrorInvalidValue;  // 2^24 rows of more than 73728 floats: 4.9 TB
     switch (op) {

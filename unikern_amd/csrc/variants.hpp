@@ -88,6 +88,12 @@ inline int rows_any_pick(long L, long C) {
   }
   return -1;  // longer rows are streamed
 }
+// The entry a plan of the family names by its tpr and nv, or, where it names none that holds the row, the pick.
+inline int rows_any_entry(int tpr, int nv, long L, long C) {
+  for (int i = 0; i < kNumRowsAny; ++i)
+    if (kRowsAny[i].tpr == tpr && kRowsAny[i].nv == nv && C <= long(tpr) * nv * 4) return i;
+  return rows_any_pick(L, C);
+}
 
 // 1-D reduce: pass-1 partial count and threads of the two-pass form, and the length up to which one
 // workgroup sums the vector in one launch instead: that takes 4.1 us up to 65536 floats and 1.5 us per
