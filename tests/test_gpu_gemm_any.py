@@ -89,6 +89,23 @@ def test_non_finite_values_stay_in_their_rows_and_columns(gpu, variant, layout):
     assert frob(got[:M - 1, :N - 1], want[:M - 1, :N - 1]) <= 1e-3
 
 
+@pytest.mark.parametrize("layout", ["TN", "NT"])
+@pytest.mark.parametrize("variant", [7, 8, 9, 10])
+@pytest.mark.parametrize("dtype, K", [("fp16", 4999), ("fp32", 2501)])
+def test_skinny_unrolled_loop(gpu, dtype, K, variant, layout):
+    # Wavefronts take the segments of k in turn, up to four of their own at a time: with 78 whole segments (156 steps
+    # in NT) each of up to sixteen runs the unrolled loop, some the one-segment remainder, one the partial segment.
+    M, N = 17, 65
+    if dtype == "fp16":
+        A, B = f16_inputs(M, N, K, 940, tn=(layout == "TN"))
+        got, R = O.f16_to_f32(run(gpu, A, B, dtype, layout, variant, off=1)), O.gemm_f16q(A, B, layout == "TN")
+    else:
+        A = O.uniform(M * K, 941, -1.0, 1.0).reshape(M, K)
+        B = O.uniform(N * K, 942, -1.0, 1.0).reshape((N, K) if layout == "TN" else (K, N))
+        got, R = run(gpu, A, B, dtype, layout, variant, off=1), O.gemm_f32(A, B, layout == "TN")
+    assert frob(got, R) <= (1e-3 if dtype == "fp16" else 1e-5)
+
+
 Q8_TILES = [11, 12, 13]  # 32x64, 64x64, 32x32
 
 
