@@ -32,3 +32,17 @@ def test_every_element(gpu, L, C):
     # A denormal numerator and its quotient each round by half of 2^-149.
     assert np.all(np.abs(Y - R)[~normal] <= 1.01 * 2.0 ** -149 + 2.0 ** -20 * R[~normal])
     assert (~normal).any() and np.all(Y[R >= 2.0 ** -148] > 0)
+
+
+@pytest.mark.parametrize("L, C", [(2000, 429), (700, 2051), (600, 5003), (400, 5003), (300, 16388)])
+def test_the_rows_sum_adds_little(gpu, L, C):
+    # A row's sum is shared by all its elements. With the threads' sums added in binary64 what is left of a row's
+    # distance is the elements' own roundings (about 2^-25 rms for the quotient and as much for v_exp_f32) and those of
+    # a thread's few additions: 4.0e-8 to 5.2e-8 measured, 8.0e-8 to 9.5e-8 with all the additions in f32.
+    X = O.normal(L * C, 50 + C, 0.0, 8.0).reshape(L, C)
+    p = gpu.Plan()
+    p.family = 2
+    Y = run_op(gpu, "softmax", X, plan=p).astype(np.float64)
+    E = np.exp(X.astype(np.float64) - X.max(axis=1, keepdims=True).astype(np.float64))
+    R = E / E.sum(axis=1, keepdims=True)
+    assert np.linalg.norm(Y - R) <= 6.5e-8 * np.linalg.norm(R)

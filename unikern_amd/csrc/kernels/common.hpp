@@ -43,6 +43,29 @@ __device__ __forceinline__ float wave_sum(float v) {
   return readlane(v, 0) + readlane(v, 32);
 }
 
+// The same in binary64 over groups of N lanes (4, 16 or the 64), the halves of each value moved alike.
+template <int N>
+__device__ __forceinline__ double lanes_sum(double v) {
+  static_assert(N == 4 || N == 16 || N == 64, "a quad, a row or the wavefront");
+  auto moved = [](double x, auto move) __attribute__((always_inline)) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_bit_cast(uint32_t, move(__builtin_bit_cast(float, (uint32_t)b)));
+    const uint32_t hi = __builtin_bit_cast(uint32_t, move(__builtin_bit_cast(float, (uint32_t)(b >> 32))));
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  };
+  v += moved(v, [](float x) { return dpp<kDppQuadXor1>(x); });
+  v += moved(v, [](float x) { return dpp<kDppQuadXor2>(x); });
+  if constexpr (N >= 16) {
+    v += moved(v, [](float x) { return dpp<kDppRowHalfMirror>(x); });
+    v += moved(v, [](float x) { return dpp<kDppRowMirror>(x); });
+  }
+  if constexpr (N == 64) {
+    v += moved(v, [](float x) { return swizzle_xor16(x); });
+    v = moved(v, [](float x) { return readlane(x, 0); }) + moved(v, [](float x) { return readlane(x, 32); });
+  }
+  return v;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp<kDppQuadXor1>(v));
   v = fmaxf(v, dpp<kDppQuadXor2>(v));

@@ -273,10 +273,11 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
 // hardware takes them in one instruction and a wavefront touches nine lines instead of eight) and the
 // one lane that holds the row's last, partial float4 going element by element. Bound by HBM. It
 // replaces three scalar passes with libm exponentials and a divide per element: RMSNorm 4096 x 4097
-// 42.1 -> 30.0 us, row-sum 1000 x 9999 14.0 -> 7.3, softmax 2048 x 5003 28.8 -> 14.4 and 64 x 70001 146 -> 15.0
-// (inputs that stay in the 256 MiB MALL), element by element no further from 64 bits (relative rms 8.4e-7
-// on both sides, which is x - max's rounding). The exponent and the quotient cost softmax 4-25% over
-// rows_kernel's (13.1 and 11.9 us, relative rms 1.2e-6 and denormals lost), a libm expf and a divide 12-60%.
+// 42.1 -> 30.0 us, row-sum 1000 x 9999 14.0 -> 7.3, softmax 2048 x 5003 28.8 -> 14.5 and 64 x 70001 147 -> 15.2
+// (inputs that stay in the 256 MiB MALL; 19.1 at 2048 x 5003 from HBM), no further from 64 bits: element by element
+// a relative rms of 8.4e-7 on both sides, which is x - max's rounding, and in 2-norm 4.7e-8 against 8.9e-8. The
+// exponent, the quotient and the sum cost softmax 4-28% over rows_kernel's arithmetic here (12.9 and 11.9 us,
+// relative rms 1.2e-6 and denormals lost), a libm expf and a divide 12-60%.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 template <int TPR, int NV, int OP>
@@ -286,7 +287,8 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
   asm volatile("" ::"s"(X), "s"(Wg), "s"(Y), "s"(L), "s"(C), "s"(eps));
   constexpr int WG = TPR < 256 ? 256 : TPR;
   constexpr int WPR = TPR / 64;
-  __shared__ float red[2][WG / 64];
+  __shared__ float red[WG / 64];
+  __shared__ double sums[WG / 64];  // softmax
   const int tid = threadIdx.x, t = tid % TPR, wave = tid >> 6;
   const int64_t row = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (WG / TPR) + tid / TPR;
   const bool active = row < L;  // rows past L are masked: every thread reaches every barrier
@@ -348,13 +350,13 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-    s = fold(wave_sum(s), red[0], add);
+    s = fold(wave_sum(s), red, add);
     if (active && t == 0) Y[row] = s;
   } else if constexpr (OP == 1) {
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
-    ss = fold(wave_sum(ss), red[0], add);
+    ss = fold(wave_sum(ss), red, add);
     const float rms = 1.0f / sqrtf(ss / (float)C + eps);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -367,14 +369,27 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
     float m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NV; ++i) m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
-    m = fold(wave_max(m), red[0], [](float a, float b) { return fmaxf(a, b); });
+    m = fold(wave_max(m), red, [](float a, float b) { return fmaxf(a, b); });
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       v[i] = f32x4{exp_sub_ulp(v[i].x, m), exp_sub_ulp(v[i].y, m), exp_sub_ulp(v[i].z, m), exp_sub_ulp(v[i].w, m)};
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
-    s = fold(wave_sum(s), red[1], add);
+    if constexpr (TPR == 64 && NV == 1) {
+      s = wave_sum(s);
+    } else {
+      // The threads' sums added in binary64: in f32 the last additions' roundings, common to the whole row, are
+      // half of the result's distance from 64 bits (8.6e-8 against 4.7e-8 at 2048 x 5003, for 1-2% of the time;
+      // rows of up to 256 floats, whose reduction shows, would pay 8%: 60000 x 83 14.1 -> 15.3 us).
+      double d = lanes_sum<64>(s);
+      if constexpr (WPR > 1) {
+        if ((tid & 63) == 0) sums[wave] = d;
+        __syncthreads();
+        d = lanes_sum<WPR>(sums[tid & (WPR - 1)]);
+      }
+      s = (float)d;
+    }
     // v / s: a product with the reciprocal, corrected by its remainder.
     const float inv = 1.0f / s;
     auto quotient = [&](float a) __attribute__((always_inline)) {
