@@ -169,25 +169,27 @@ int uk_solve(const char* hcs_json, const uk_op_desc* d, uk_plan* out, char* log,
  * uk_launch: enqueue the op on `stream` over caller-owned device buffers.
  *   gemm f32/f16:  in[0]=A, in[1]=B (layout NT: [K][N]; TN: [N][K]); out=C [M][N] (same dtype)
  *   gemm q8_0 TN:  in[0]=X f16 [M][K], in[1]=W blocks (N rows of K/32 blocks); out=Y f32 [M][N]
- *                  (X 16-byte aligned, Y 4-byte; W 16-byte aligned where K is a multiple of 256,
- *                  which every variant the solver picks there copies in 16-byte units, else 4-byte)
+ *                  (X 16-byte aligned, Y 4-byte; W 16-byte aligned where K is a multiple of 256, which
+ *                  the split-k and one-row kernels copy in 16-byte units (tiles of more than 16 rows take
+ *                  4-byte there too), else 4-byte)
  *   conv NT:       in[0]=X [H][W][C], in[1]=Wt [Oc][Kh][Kw][C] (, in[2]=scale[Oc]); out=Y [Oc][Ho][Wo]
  *   conv NCHW:     in[0]=X [N][C][H][W], in[1]=W [Oc][C][Kh][Kw] (, in[2]=scale[Oc]); out=Y [N][Oc][Ho][Wo]
  *   reduce [L]:    in[0]=X; out=Y[1]           reduce [L,C]: in[0]=X; out=Y[L] (row sums)
  *   softmax:       in[0]=X; out=Y               rmsnorm: in[0]=X, in[1]=W[C]; out=Y
  *   channelscale:  in[0]=X, in[1]=S[C]; out=Y
  * plan may be NULL (solved against the built-in MI355X description).
- * Allocates nothing. The 1-D reduce keeps its pass-1 partials (8 KiB) in a static device array,
- * one per GPU, held until the process ends; a 1-D reduce waits (hipStreamWaitEvent on one event
- * per GPU) for the previous one enqueued on that GPU through uk_launch or uk_launch_n, whatever
- * its stream, so two never share the partials at once. That wait is an event recorded outside
- * any graph: callers under HIP graph capture use uk_launch_noalloc. */
+ * Allocates nothing. A 1-D reduce of more than 262144 floats keeps its pass-1 partials (8 KiB) in a
+ * static device array, one per GPU, held until the process ends; it waits (hipStreamWaitEvent on
+ * one event per GPU) for the previous one enqueued on that GPU through uk_launch or uk_launch_n,
+ * whatever its stream, so two never share the partials at once. That wait is an event recorded
+ * outside any graph: callers under HIP graph capture use uk_launch_noalloc. Shorter ones run in one
+ * launch without partials or events. */
 int uk_launch(const uk_op_desc* d, const uk_plan* plan, const void* const* in, int32_t n_in, void* out,
               void* stream);
 /* uk_launch that allocates nothing: no counterpart in the reference; for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). Same arguments, kernels and results as uk_launch. The scratch a launch
- * needs beyond its inputs and output (the 1-D reduce's 8 KiB of pass-1 partials) comes from a
+ * needs beyond its inputs and output (a long 1-D reduce's 8 KiB of pass-1 partials) comes from a
  * static 1 MiB device array, one per GPU, held until the process ends; its device address is
  * looked up on the first call on each device. A launch needing more is refused (class 2).
  * Every call on one GPU shares that array and nothing in it needs to start at zero: calls that

@@ -136,9 +136,9 @@ std::string support_gap(const KmlTree& t);
 enum class Family : int {
   None = 0,
   Rows = 1,          // row-sum / rmsnorm / softmax, row held in registers
-  RowsStream = 2,    // same ops, any row length, row streamed twice
+  RowsStream = 2,    // same ops, any row length: in registers up to 73728 floats, streamed beyond
   ChannelScale = 3,  // standalone elementwise channelscale
-  Reduce1D = 4,      // scalar sum, two deterministic passes
+  Reduce1D = 4,      // scalar sum, deterministic: one workgroup, or two passes beyond 262144 floats
   GemmF16 = 5,       // MFMA f16 GEMM, LDS-staged, f32 accumulate
   GemmGeneric = 6,   // MFMA GEMM for any shape/layout (f16 or f32)
   ConvIgemm = 7,     // implicit-GEMM conv on f32 MFMA, fused channelscale

@@ -16,6 +16,10 @@
 // channel pair re-read the same few cache lines from L1; the next channel pair's gathers are
 // issued before the current pair's MFMAs. Padding taps read as zero.
 //
+// The solver takes conv_igemm_kernel and conv_tile_kernel for few shapes now: conv_any.hip, whose tiles gather
+// an input once, is faster at nearly all of them. They serve small launches (2x2 kernels, 1x1 over a few
+// pixels), images of 2 GiB and more, which conv_any's 32-bit offsets do not cover, and plans that name them.
+//
 // Layouts: NCHW (X[N][C][H][W], W[Oc][C][Kh][Kw], Y[N][Oc][Ho][Wo], zero padding, stride) and
 // the reference's NT conv (X[H][W][C], Wt[Oc][Kh][Kw][C], Y[Oc][Ho][Wo], valid padding,
 // src/reference.cpp:6-22).

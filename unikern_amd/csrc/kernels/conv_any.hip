@@ -12,11 +12,12 @@
 //
 // Why: the gathering kernels (conv_igemm, conv_tile) load every input element straight into the MFMA
 // operands of each wavefront that needs it, one load per MFMA; here a tile's input is loaded once
-// and an element costs one load instead of one per 32 output channels. Bound by the f32 MFMA rate of
-// the busiest CU (dependent 16x16x4 chains of two to four wavefronts per SIMD) and, in NCHW, by the
-// gather's loads. HWC 256x256x32, 3x3, 64 channels: 89.7 -> 26.9 us (88 TFLOP/s, 56% of the f32 MFMA
-// peak); NCHW 8x64x56x56 stride 2 55.8 -> 17.2, 8x64x56x56 1x1 to 256 57.8 -> 20.2, 8x256x14x14 3x3
-// 183 -> 54.8, 4x3x112x112 7x7 stride 2 36.2 -> 10.9. NCHW 3x3 stride 1 of aligned rows stays on the
+// and an element costs one load instead of one per 32 output channels. Bound by the f32 MFMA of the CU (0.62 of
+// its cycles at HWC 256x256x32, 14 of 16 wavefronts resident: the fill at the start, when every tile
+// builds its table and loads, and the stores at the end are the rest) and, in NCHW, by the gather's loads.
+// HWC 256x256x32, 3x3, 64 channels: 89.7 -> 26.5 us (90 TFLOP/s, 57% of the f32 MFMA
+// peak; 29.0 from HBM); NCHW 8x64x56x56 stride 2 53.8 -> 17.3, 8x64x56x56 1x1 to 256 56.2 -> 20.7, 8x256x14x14 3x3
+// 174 -> 54.5, 4x3x112x112 7x7 stride 2 35.9 -> 11.9. NCHW 3x3 stride 1 of aligned rows stays on the
 // kernels that stage whole input rows (conv_lds16: 20.7 us at 8x64x56x56, 36.0 here).
 #include "../launch.hpp"
 #include "../variants.hpp"

@@ -18,15 +18,18 @@
 //   do, and B stored [K][N] is transposed on its way (v_perm on pairs of k). With S > 1, S groups of
 //   wavefronts multiply S consecutive 128-byte segments and add their sums in LDS at the end: small
 //   grids then have S times the loads in flight. Bound by load latency below about two workgroups per
-//   CU and by the matrix pipe of two wavefronts per SIMD above.
+//   CU; above, no pipe is full (256x192 at 1000x11008x4096: matrix cores 0.50 of a busy CU's cycles, LDS 0.39;
+//   row-major B at 512x9728x2560: 0.36, LDS 0.48 of which the transposing stores' conflicts 0.15, vector ALU
+//   0.32): a step's stores, fragment reads and MFMAs follow each other in the two wavefronts of a SIMD.
 // gemm_skinny_*_kernel: 16-32 rows of A. Wavefronts split k, each lane loads its fragments of both
 //   operands straight into registers (no LDS, no barrier until the partial sums are added), several
-//   steps' loads in flight. Bound by the stream of B.
+//   steps' loads in flight. Bound by the vector cache's tag lookups (0.89 a cycle at 16x11008x4096: the lanes of a
+//   load are 16 rows apart), then the stream of B.
 //
 // Measured against the bounds-checked 64x64x16 kernel these replaced (element loads, two barriers per
 // 16 k), one box, inputs rotating over three sets: f16 TN 1000x11008x4096 2667 -> 96.8 us (932
 // TFLOP/s; 256x192), 16x11008x4096 251 -> 23.9 us (3.8 TB/s; skinny), f16 NT 512x9728x2560 440 ->
-// 47.0 us (543 TFLOP/s; 256x128), f32 NT 1000^3 131 -> 24.8 us (81 TFLOP/s; 64x64 in two k groups),
+// 46.8 us (545 TFLOP/s; 256x128), f32 NT 1000^3 131 -> 24.8 us (81 TFLOP/s; 64x64 in two k groups),
 // and against 64 bits the f32 sums are no further off (4.0e-7 against 5.7e-7).
 #include "../launch.hpp"
 #include "../variants.hpp"

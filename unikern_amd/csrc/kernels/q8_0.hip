@@ -473,12 +473,12 @@ __global__ void __launch_bounds__(WAVES * 64)
 // per k group, operands staged through registers a whole round ahead as in gemm_any.hip. Each block's
 // 16x16x32 MFMA starts from zero and its four sums are scaled and added in f32 (X first: a lane's four
 // sums belong to one weight row, so it needs one scale), the same arithmetic as above.
-// Bound: per block and 16x16 tile the four multiply-adds take as long on the vector ALU as the MFMA on
-// the matrix cores, and the conversion comes on top; both share the time with LDS (half of the cycles
-// at 64x64) and the texture cache's tag lookups. 512x4096x4096: 85.4 -> 44.3 us (388 TFLOP/s),
-// 512x11008x4096 277 -> 126, 64x11008x4096 41.1 -> 22.4; up to 16 rows keep the kernels above. (Two k
-// groups in 64x64 tiles took 40 and 110 us, 128x128 tiles of one group 90 at 512x11008x4096, with
-// the sums of one chain; with as many chains as here they need more registers and are slower.)
+// Bound: the vector ALU (conversion and the four multiply-adds per block and 16x16 tile: 0.43 of a busy CU's
+// cycles at 512x4096x4096), LDS (0.44, a fifth of it conflicts) and the MFMAs (0.14) take their turns between
+// the barriers of one workgroup of sixteen wavefronts, and add up to one. 512x4096x4096: 85.4 -> 43.6-44.7 us
+// (390 TFLOP/s; 51.3 from HBM), 512x11008x4096 276 -> 131, 64x11008x4096 41.0 -> 22.5; up to 16 rows keep the
+// kernels above. (Tiles of 64x64 in two k groups and of 128x128 took less with one chain per output and no
+// blocks; with as many chains as was then needed they took more registers and were slower.)
 template <int BM, int BN, int WM, int WN, int S>
 struct Q8TileCfg {
   static constexpr int kGroup = WM * WN * 64;  // threads of one k group
@@ -530,9 +530,9 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   const int wrow = tg >> 2, wb = (tg >> 1) & 1, wh = tg & 1;
   // A pair is 17 dwords: d0 in the low half of dword 0, the even block's quants from byte 2, d1 in the
   // high half of dword 8, the odd block's quants from dword 9. Each lane loads whole dwords: 16 bytes
-  // at dword 0, 4, 9 or 13 and the dword 4, 8, 8 or 13 that completes them (unaligned 16-byte loads
-  // of the quants and 2-byte loads of the scales kept the texture cache busy all the time: 95.7k tag
-  // lookups per CU in a launch of 98k cycles, 62k now).
+  // at dword 0, 4, 9 or 13 and the dword 4, 8, 8 or 13 that completes them (unaligned 16-byte loads of the
+  // quants and 2-byte loads of the scales look up more cache tags; these make 73k per CU in 115k busy cycles at
+  // 512x4096x4096).
   const int wext = wb ? (wh ? 0 : -4) : 16;
   const int wshift = wb ? 0 : 2;
   const int p0 = kh < npairs ? kh : npairs - 1;

@@ -56,7 +56,7 @@ constexpr RowsVariant kRowsVariants[] = {
 constexpr int kNumRowsVariants = sizeof(kRowsVariants) / sizeof(kRowsVariants[0]);
 
 // Standalone channelscale in the grouped-store row form (one wavefront per row of at most 4096
-// floats, more than half of its lanes busy); other shapes take the float4 grid-stride kernel.
+// floats, more than half of its lanes busy).
 inline bool channelscale_rows_form(long L, long C) { return C % 4 == 0 && C > 2048 && C <= 4096 && L <= 0x7fffffffL; }
 // Other shapes go as a flat array (channelscale_flat_kernel): workgroups of 4096 floats, or of 1024 where
 // there would be fewer than two of those per CU. Rows of 2049-4096 floats in multiples of 4 keep the row
@@ -158,7 +158,8 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // share of the CU's time (work_f16 / work_f32, times nt_factor where B is [K][N], times `unaligned`
 // where the rows of B are not whole 16-byte chunks), tail the fold and stores in iterations. Fitted
 // over 515 shapes drawn from M 1-4096, N 64-11008, K 64-4096 (every variant measured at each, both
-// types and layouts): the pick's time is about 2% over the fastest variant's on average. Whatever the
+// types and layouts) whose inputs stayed in the MALL: the pick's time is about 2% over the fastest variant's
+// on average (26% at 16x11008x4096 TN: 23.4 us for variant 7 where variant 2 takes 17.0). Whatever the
 // sum says, no variant has sustained more than kGemmAnyPeakF16 / F32 of the matrix-core peak.
 // The 64x64 variant 0 is the one any shape falls back to; a product of a single tile of it (M, N <= 64) is offered
 // variant 7 in its place, whose 16-row workgroups spread it over CUs (64x64x96 f32: 3.9 against 5.1 us).
@@ -168,7 +169,7 @@ constexpr int kNumGemmF16Variants = sizeof(kGemmF16Variants) / sizeof(kGemmF16Va
 // 3637x2887x3584 98 -> 86; picked at five of 49 drawn TN shapes and the fastest at each. For B [K][N] its
 // three chunks per thread do not split into pairs of k, and the 128x192 tile that would, in two k groups,
 // gained 1% at best over 256x128 there (46.5 against 46.8 us at 512x9728x2560): not compiled.
-// id: the plan's variant number (1 is gemm_f32_kernel). resident: workgroups per CU by LDS and registers.
+// id: the plan's variant number (1 is gemm_f32_kernel). resident: the workgroups per CU the costs were fitted with.
 struct GemmAnyVariant {
   int id, bm, bn, wm, wn, ks, mt, nt, waves, unroll, resident, f16_only;
   double lat_us, work_f16, work_f32, nt_factor, fixed_us, tail, unaligned;
@@ -333,7 +334,8 @@ inline bool conv_l16_supported(bool nchw, long kh, long kw, long stride, long pa
 // plan's variant number is kNumConvVariants + index. Cost: fixed_us + (32 ks-deep steps of k + tail) *
 // sum over rounds of max(lat, n * work), n the workgroups a CU holds (the form of kGemmAnyVariants'
 // cost), fitted over 220 drawn shapes (7-256 pixels a side, 3-256 channels, kernels of 1, 3 and 5): the
-// pick is 1.2% over the fastest on average. work: NCHW, HWC with C a multiple of 4 (16-byte loads), HWC.
+// pick is 1.2% over the fastest on average. resident is what the fit took (a CU holds four of the first
+// variant: 14.2 of 16 wavefronts counted at 256x256x32). work: NCHW, HWC with C a multiple of 4 (16-byte loads), HWC.
 struct ConvAnyVariant {
   int bm, bn, wm, wn, ks, resident;
   double lat_us, lat_vec_us, work_nchw, work_vec, work_hwc, fixed_us, tail;
