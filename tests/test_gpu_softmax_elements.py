@@ -38,7 +38,7 @@ def test_every_element(gpu, L, C):
 def test_the_rows_sum_adds_little(gpu, L, C):
     # A row's sum is shared by all its elements. With the threads' sums added in binary64 what is left of a row's
     # distance is the elements' own roundings (about 2^-25 rms for the quotient and as much for v_exp_f32) and those of
-    # a thread's few additions: 4.0e-8 to 5.2e-8 measured, 8.0e-8 to 9.5e-8 with all the additions in f32.
+    # a thread's few additions: 3.2e-8 to 4.3e-8 measured, 8.0e-8 to 9.5e-8 with all the additions in f32.
     X = O.normal(L * C, 50 + C, 0.0, 8.0).reshape(L, C)
     p = gpu.Plan()
     p.family = 2

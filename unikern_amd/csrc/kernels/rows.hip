@@ -14,7 +14,7 @@
 // y = exp(x - max) / sum(exp(x - max)), in rows_kernel as 2^((x - max) log2 e) * (1 / sum) on v_exp_f32
 // (exp_sub below): within about 2e-6 of the reference wherever the 1e-5 relative gate can see an
 // element, and a fifth of the vector instructions of a libm exp and a divide per element; in
-// rows_any_kernel to an ulp (exp_sub_ulp and a corrected quotient), as in the libm form of
+// rows_any_kernel to an ulp (exp_sub_2p64 and a corrected quotient), as in the libm form of
 // rows_stream_kernel.
 #include <math.h>
 
@@ -53,17 +53,20 @@ __device__ __forceinline__ void st4(f32x4* p, f32x4 v) {
 constexpr float kLog2eF = 1.44269502f;  // log2(e) rounded to binary32
 __device__ __forceinline__ float exp_sub(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kLog2eF); }
 
-// e^(x - m) to about an ulp of the subtraction's result, as a libm expf: (x - m) log2 e = n + r with n an
+// 2^64 e^(x - m) to about an ulp of the subtraction's result, as a libm expf: (x - m) log2 e = n + r with n an
 // integer and |r| <= 1/2, the product's rounding and the binary32 log2(e)'s kept in r by two fused
-// multiply-adds, and 2^n applied by an exponent add that reaches the denormals. Below -104 the result is 0
-// (under half the smallest denormal), which is also what -inf gives; NaN stays NaN.
+// multiply-adds. n is rounded off by the addition of 1.5 2^23, whose low bits then hold it and are shifted into the
+// factor 2^(n + 64). The row's sum carries the same 2^64, which leaves with the quotient, so that numerators
+// below 2^-126 lose nothing. n stops at -160, where the element is 0 (-inf among them); NaN stays NaN in r.
 constexpr float kLog2eLoF = 1.92596303e-8f;  // log2(e) - kLog2eF
-__device__ __forceinline__ float exp_sub_ulp(float x, float m) {
+constexpr float kRoundF = 12582912.f;        // 1.5 2^23
+__device__ __forceinline__ float exp_sub_2p64(float x, float m) {
   const float d = x - m;
-  const float n = __builtin_rintf(d * kLog2eF);
+  const float t = fmaxf(__builtin_fmaf(d, kLog2eF, kRoundF), kRoundF - 160.f);
+  const float n = t - kRoundF;
   const float r = __builtin_fmaf(d, kLog2eLoF, __builtin_fmaf(d, kLog2eF, -n));
-  const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(r), (int)n);
-  return d < -104.f ? 0.f : e;
+  const float scale = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, t) << 23) + (uint32_t(127 + 64) << 23));
+  return __builtin_amdgcn_exp2f(r) * scale;
 }
 
 // TPR threads own one row at a time and each keeps NV float4 of it in registers; a workgroup
@@ -273,15 +276,15 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
 // hardware takes them in one instruction and a wavefront touches nine lines instead of eight) and the
 // one lane that holds the row's last, partial float4 going element by element. Bound by HBM. It
 // replaces three scalar passes with libm exponentials and a divide per element: RMSNorm 4096 x 4097
-// 42.1 -> 30.0 us, row-sum 1000 x 9999 14.0 -> 7.3, softmax 2048 x 5003 28.8 -> 14.5 and 64 x 70001 147 -> 15.2
-// (inputs that stay in the 256 MiB MALL; 19.1 at 2048 x 5003 from HBM), no further from 64 bits: element by element
-// a relative rms of 8.4e-7 on both sides, which is x - max's rounding, and in 2-norm 4.7e-8 against 8.9e-8. The
-// exponent, the quotient and the sum cost softmax 4-28% over rows_kernel's arithmetic here (12.9 and 11.9 us,
+// 42.1 -> 30.0 us, row-sum 1000 x 9999 14.0 -> 7.3, softmax 2048 x 5003 28.8 -> 14.3 and 64 x 70001 147 -> 14.7
+// (inputs that stay in the 256 MiB MALL; 19.3 at 2048 x 5003 from HBM), no further from 64 bits: element by element
+// a relative rms of 8.4e-7 on both sides, which is x - max's rounding, and in 2-norm 3.6e-8 against 8.9e-8. The
+// exponent, the quotient and the sum cost softmax 4-30% over rows_kernel's arithmetic here (12.9 and 11.9 us,
 // relative rms 1.2e-6 and denormals lost), a libm expf and a divide 12-60%.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 template <int TPR, int NV, int OP>
-__global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
+__global__ void __launch_bounds__(TPR < 256 ? 256 : TPR, OP == 2 && NV <= 8 ? 8 : TPR == 1024 ? 4 : 2)
     rows_any_kernel(const float* __restrict__ X, const float* __restrict__ Wg, float* __restrict__ Y, int L, int C,
                     float eps) {
   asm volatile("" ::"s"(X), "s"(Wg), "s"(Y), "s"(L), "s"(C), "s"(eps));
@@ -335,9 +338,12 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
   };
   static_assert(WPR == 1 || WG == TPR, "a workgroup of several wavefronts per row holds one row");
   auto add = [](float a, float b) { return a + b; };
+  // The stores' indices are computed again: kept from the loads they cost a register each (56 bytes of scratch at
+  // 18 float4 a thread).
+  int ts = t;
   auto put = [&](int i, f32x4 o) __attribute__((always_inline)) {
     float* y = Y + row * (int64_t)C;
-    const int j = i * TPR + t;
+    const int j = i * TPR + ts;
     if (active && j < C4) {
       *reinterpret_cast<f32x4_any*>(y + 4 * j) = o;
     } else if (active && j == C4 && tail) {
@@ -373,29 +379,31 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR)
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      v[i] = f32x4{exp_sub_ulp(v[i].x, m), exp_sub_ulp(v[i].y, m), exp_sub_ulp(v[i].z, m), exp_sub_ulp(v[i].w, m)};
+      v[i] = f32x4{exp_sub_2p64(v[i].x, m), exp_sub_2p64(v[i].y, m), exp_sub_2p64(v[i].z, m), exp_sub_2p64(v[i].w, m)};
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
+    // The reciprocal in two parts: a product with it is a quotient to half an ulp, denormals included.
+    float inv, inv_lo;
     if constexpr (TPR == 64 && NV == 1) {
       s = wave_sum(s);
+      inv = 1.0f / s;
+      inv_lo = __builtin_fmaf(-s, inv, 1.0f) * inv;
     } else {
       // The threads' sums added in binary64: in f32 the last additions' roundings, common to the whole row, are
-      // half of the result's distance from 64 bits (8.6e-8 against 4.7e-8 at 2048 x 5003, for 1-2% of the time;
+      // half of the result's distance from 64 bits (8.6e-8 against 4.0e-8 at 2048 x 5003, for 1-2% of the time;
       // rows of up to 256 floats, whose reduction shows, would pay 8%: 60000 x 83 14.1 -> 15.3 us).
-      double d = lanes_sum<64>(s);
+      double sum = lanes_sum<64>(s);
       if constexpr (WPR > 1) {
-        if ((tid & 63) == 0) sums[wave] = d;
+        if ((tid & 63) == 0) sums[wave] = sum;
         __syncthreads();
-        d = lanes_sum<WPR>(sums[tid & (WPR - 1)]);
+        sum = lanes_sum<WPR>(sums[tid & (WPR - 1)]);
       }
-      s = (float)d;
+      const double q = 1.0 / sum;
+      inv = (float)q;
+      inv_lo = (float)(q - (double)inv);
     }
-    // v / s: a product with the reciprocal, corrected by its remainder.
-    const float inv = 1.0f / s;
-    auto quotient = [&](float a) __attribute__((always_inline)) {
-      const float q = a * inv;
-      return __builtin_fmaf(__builtin_fmaf(-q, s, a), inv, q);
-    };
+    asm volatile("" : "+v"(ts));
+    auto quotient = [&](float a) __attribute__((always_inline)) { return __builtin_fmaf(a, inv, a * inv_lo); };
 #pragma unroll
     for (int i = 0; i < NV; ++i) put(i, f32x4{quotient(v[i].x), quotient(v[i].y), quotient(v[i].z), quotient(v[i].w)});
   }
