@@ -248,9 +248,9 @@ __global__ void __launch_bounds__(WM* WN* S * 64, 4)
     store.template operator()<true>(0);
     lds_barrier();
     multiply(0);
+    fold();
     lds_barrier();
   }
-  fold();
 
   if constexpr (S > 1) {
     f32x4* red = reinterpret_cast<f32x4*>(lds);
