@@ -402,10 +402,6 @@ constexpr double kActBytesPerUsPerCu = 100e3;  // activation bytes per us per CU
 // row family's 2 us figure, which covers a cold start, overstates it here).
 constexpr double kQ8LatencyUs = 1.0;
 
-// Tiles are taken only where they are cheaper by more than the fits agree on (359x320x4352: 11.8 against
-// 11.9 us predicted, 12.7 against 11.1 measured).
-constexpr double kQ8TileMargin = 1.03;
-
 // A launch of `wgs` workgroups of `iters` k rounds each for more than 16 activation rows.
 double q8_many_us(const Hcs& h, const Q8Many& v, int64_t wgs, int64_t iters, int resident) {
   const double work = v.work / mfma_clock_scale(h);
@@ -418,10 +414,9 @@ double q8_many_us(const Hcs& h, const Q8Many& v, int64_t wgs, int64_t iters, int
 // More than 16 rows: which of the split-k kernels stand beside the tiles. A wavefront of theirs sums its
 // blocks of all rounds in one chain, so a variant is not offered if its chain is longer than that of the
 // variant the weight stream's cost ranks first: eight wavefronts for its sixteen beyond K = 2048 round off
-// 10-13% more against 64 bits and are 3-9% slower (72x64x9536: 14.8 against 13.5 us). With chains no longer,
-// the costs fitted below decide against the tiles, but not between split-k kernels of several rounds (375x250x10752:
-// the one they rank first 27.3, the stream's 22.2 us) nor for fewer wavefronts at one round (they are 1.3 us
-// high for sixteen there: 5.8 against 4.5 us measured at K <= 2048): there the stream's first takes the cost.
+// 10-13% more against 64 bits (72x64x9536: 14.8 against 13.5 us as well). Where the first takes several rounds, the
+// costs fitted below decide between it and the tiles only, not among split-k kernels (375x250x10752: the one
+// they rank first 27.3, the stream's 22.2 us); within one round, where chains are the same, they decide.
 void keep_q8_chains(std::vector<Cand>* cs, const std::vector<double>& stream_cost, int64_t npairs, SolveLog* log) {
   size_t first = 0;
   for (size_t i = 1; i < cs->size(); ++i)
@@ -433,8 +428,7 @@ void keep_q8_chains(std::vector<Cand>* cs, const std::vector<double>& stream_cos
     return (npairs + v.waves * v.pairs - 1) / (v.waves * v.pairs) * v.pairs;
   };
   const int64_t longest = chain((*cs)[first]);
-  const int waves = (*cs)[first].plan.split_k;
-  const bool rounds = npairs > waves * kQ8Variants[(*cs)[first].plan.variant].pairs;
+  const bool rounds = npairs > (*cs)[first].plan.split_k * kQ8Variants[(*cs)[first].plan.variant].pairs;
   double cost = (*cs)[first].cost;
   std::vector<Cand> kept;
   for (size_t i = 0; i < cs->size(); ++i) {
@@ -442,7 +436,7 @@ void keep_q8_chains(std::vector<Cand>* cs, const std::vector<double>& stream_cos
     if (i == first) continue;
     if (chain(c) > longest) {
       reject(log, c.plan.key + " violates chain of blocks <= " + std::to_string(2 * longest));
-    } else if (rounds || c.plan.split_k < waves) {
+    } else if (rounds) {
       cost = std::min(cost, c.cost);
     } else {
       kept.push_back(c);
@@ -606,7 +600,7 @@ std::optional<Plan> solve_q8(const Hcs& h, const KmlTree& t, const Shape& s, Sol
     c.plan.key = key;
     c.plan.why = std::to_string(c.plan.grid) + " tiles, weights converted once per " + std::to_string(v.bm) + " rows";
     c.cost = std::max(launch_us(h) + double(w.bytes) / (hbm_gbps(h) * 1e3 * kStreamEff),
-                      kQ8TileMargin * q8_many_us(h, v.many, c.plan.grid, (npairs + v.ks - 1) / v.ks, v.resident));
+                      q8_many_us(h, v.many, c.plan.grid, (npairs + v.ks - 1) / v.ks, v.resident));
     cs.push_back(std::move(c));
   }
   return pick(cs, "q8_0", log, err);

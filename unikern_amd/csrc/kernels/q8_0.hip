@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(WAVES * 64)
 // sums belong to one weight row, so it needs one scale), the same arithmetic as above.
 // Bound: the vector ALU (conversion and the four multiply-adds per block and 16x16 tile: 0.43 of a busy CU's
 // cycles at 512x4096x4096), LDS (0.44, a fifth of it conflicts) and the MFMAs (0.14) take their turns between
-// the barriers of one workgroup of sixteen wavefronts, and add up to one. 512x4096x4096: 85.4 -> 43.6-44.7 us
+// the barriers of one workgroup of sixteen wavefronts, and add up to one. 512x4096x4096: 85.4 -> 43.6-45.0 us
 // (390 TFLOP/s; 51.3 from HBM), 512x11008x4096 276 -> 131, 64x11008x4096 41.0 -> 22.5; up to 16 rows keep the
 // kernels above. (Tiles of 64x64 in two k groups and of 128x128 took less with one chain per output and no
 // blocks; with as many chains as was then needed they took more registers and were slower.)
@@ -592,11 +592,11 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   };
   const int fi = lane & 15, fg = lane >> 4;
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Summation in blocks: `part` runs over the eight blocks of four rounds, then goes into `acc`. Its
-  // roundings grow with half the chain, those of `acc` with a sixteenth of a k group's length, so the sum
-  // rounds off less than the split-k kernels' at any K: one chain per wavefront there (8 or 16 chains),
-  // and one fused multiply-add per block in both (a sum of even and a sum of odd blocks, as many registers,
-  // cost a short K one more rounding: 4.6e-8 against 4.1e-8 at K = 64).
+  // Summation in blocks: `part` runs over the four blocks of two rounds, then goes into `acc`. The sum rounds off
+  // less than the split-k kernels' (one chain per wavefront, 8 or 16 of them) at any K but 128, where it is 1.02
+  // times as far from 64 bits: 0.96 of the sixteen-wavefront kernel's error at K <= 1024, 0.89 to 4096, 0.875
+  // beyond. A sum of even and a sum of odd blocks over all of K, as many registers, was 1.11 times as far at K = 64-128
+  // (one rounding more) and 1.04-1.09 times at K above 7000.
   f32x4 acc[FM][FN], part[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -662,9 +662,8 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   for (int t = 0; t * S < npairs; t += 2) {
     round(I0{}, t);
     round(I1{}, t + 1);
-    if (t & 2) fold();
+    fold();
   }
-  fold();
   if constexpr (S > 1) {
     f32x4* red = reinterpret_cast<f32x4*>(lds);
     if (kh > 0) {
