@@ -122,3 +122,18 @@ def test_pixels_of_a_1x1_conv(gpu):
     for at in (0, n // 2, n - 4096):
         assert (read(gpu, yb, at * 4, 4096) == want).all()
     assert guard(gpu, yb, n * 4)
+
+
+@pytest.mark.parametrize("variant", [7, 0])
+def test_gemm_tiles(gpu, variant):
+    # 1.3 M tiles of 16x16, or of 64x64: the fold into y starts at 2^20 of them. Small integers: exact.
+    M, N = (4194240, 80) if variant == 7 else (4194240, 1025)
+    a = (np.arange(M, dtype=np.int64) * 7 % 13).astype(np.float16)
+    b = (np.arange(N) % 11).astype(np.float16)
+    p = gpu.Plan()
+    p.family, p.variant = 6, variant
+    ab, bb, cb = gpu.DeviceBuffer.from_array(a), gpu.DeviceBuffer.from_array(b), output(gpu, M * N * 2)
+    gpu.launch(gpu.make_desc("gemm", [M, N, 1], dtype="fp16", layout="TN"), [ab, bb], cb, plan=p)
+    for r in (0, M // 2 + 3, M - 1):
+        assert np.array_equal(read(gpu, cb, r * N * 2, N, np.float16), a[r] * b)
+    assert guard(gpu, cb, M * N * 2)

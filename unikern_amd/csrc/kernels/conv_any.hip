@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(WM* WN* S * 64, 4)
   const int tg = tid - kh * Cfg::kGroup;
 
   const int per_image = a.tiles_m * a.tiles_n;
-  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int id = folded_id();
   if (id >= a.tiles) return;
   const int image = id / per_image, in_image = id - image * per_image;
   const int m0 = in_image % a.tiles_m * BM, n0 = in_image / a.tiles_m * BN;

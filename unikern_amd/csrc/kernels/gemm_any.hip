@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   // Workgroup i runs on XCD i % 8: give each XCD a contiguous range of tiles (the first G % 8 XCDs
   // one more), walked in groups of 4 tile rows.
   const int G = tiles_m * tiles_n;
-  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int id = folded_id();
   if (id >= G) return;
   const int xcd = id & 7, per = G >> 3, rem = G & 7;
   const int lin = xcd * per + (xcd < rem ? xcd : rem) + (id >> 3);
@@ -378,7 +378,7 @@ __global__ void __launch_bounds__(W * 64)
   __shared__ f32x4 red[W * MT * NT * 64];
   const int lane = threadIdx.x & 63, fi = lane & 15, fg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int id = folded_id();
   if (id >= gm * gn) return;
   const int n0 = id % gn * 16 * NT, m0 = id / gn * 16 * MT;
   const T* arow[MT];
@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(W * 64)
   __shared__ f32x4 red[W * MT * 4 * 64];
   const int lane = threadIdx.x & 63, fi = lane & 15, fg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int id = folded_id();
   if (id >= gm * gn) return;
   const int n0 = id % gn * 64, m0 = id / gn * 16 * MT;
   const int n = n0 + 4 * fi;

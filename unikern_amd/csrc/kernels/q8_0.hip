@@ -509,7 +509,7 @@ __global__ void __launch_bounds__(WM* WN* S * 64)
   const int tg = tid - kh * Cfg::kGroup;
 
   const int G = tiles_m * tiles_n;
-  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int id = folded_id();
   if (id >= G) return;
   const int xcd = id & 7, per = G >> 3, rem = G & 7;
   const int lin = xcd * per + (xcd < rem ? xcd : rem) + (id >> 3);

@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(TPR < 256 ? 256 : TPR, OP == 2 && NV <= 8 ? 8 
   __shared__ float red[WG / 64];
   __shared__ double sums[WG / 64];  // softmax
   const int tid = threadIdx.x, t = tid % TPR, wave = tid >> 6;
-  const int64_t row = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (WG / TPR) + tid / TPR;
+  const int64_t row = (int64_t)folded_id() * (WG / TPR) + tid / TPR;
   const bool active = row < L;  // rows past L are masked: every thread reaches every barrier
   const float* x = X + (active ? row : 0) * (int64_t)C;
   const int tail = C & 3, C4 = C >> 2;
@@ -467,7 +467,7 @@ __global__ void __launch_bounds__(256)
     channelscale_flat_kernel(const float* __restrict__ X, const float* __restrict__ S, float* __restrict__ Y, int64_t n,
                              unsigned C) {
   asm volatile("" ::"s"(X), "s"(S), "s"(Y), "s"(n), "s"(C));
-  const int64_t base = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (U * 1024);
+  const int64_t base = (int64_t)folded_id() * (U * 1024);
   if (base >= n) return;
   const int64_t left = n - base;
   const int here = left < U * 1024 ? (int)left : U * 1024;

@@ -7,15 +7,15 @@
 #include <cstdint>
 
 #include "host/uk_core.hpp"
+#include "variants.hpp"
 
 namespace uk {
 
 // The grid of `wgs` workgroups (at most 2^31 - 1): a grid dimension holds fewer than 2^32 work items, so more
-// than 2^20 workgroups fold into y. A kernel launched so flattens its id (blockIdx.y * gridDim.x +
-// blockIdx.x) and returns where that is past the last workgroup.
+// than kFoldedRow workgroups fold into y. A kernel launched so takes its id from kern::folded_id() and returns
+// where that is past the last workgroup.
 inline dim3 folded_grid(int64_t wgs) {
-  constexpr int64_t kRow = 1 << 20;
-  return wgs <= kRow ? dim3((unsigned)wgs) : dim3((unsigned)kRow, (unsigned)((wgs + kRow - 1) / kRow));
+  return wgs <= kFoldedRow ? dim3((unsigned)wgs) : dim3(kFoldedRow, (unsigned)((wgs + kFoldedRow - 1) / kFoldedRow));
 }
 
 enum class RowOp : int { Sum = 0, RmsNorm = 1, Softmax = 2 };

@@ -8,6 +8,7 @@ namespace uk {
 // Work items of one grid dimension. The runtime takes a launch of more without an error and runs what is
 // left of the number modulo 2^32.
 constexpr long kGridDimItems = 0xffffffffL;
+constexpr int kFoldedRow = 1 << 20;  // workgroups in x of a grid that folds into y
 inline bool grid_dim_holds(long workgroups, int threads) { return workgroups <= kGridDimItems / threads; }
 
 // Row family (row-sum, RMSNorm, softmax with the row held in registers).
